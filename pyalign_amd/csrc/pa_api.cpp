@@ -882,16 +882,92 @@ void stage_payload(pa_solver &s, const Input &in, hipStream_t st, const void *&c
 }
 
 
-// General gap costs (Waterman-Smith-Beyer): one workgroup per problem, no
-// strip schedule.  The kernel leaves D, S and the traceback codes of every
-// cell in device memory; all-optimal enumeration and Solution matrices read
-// them on the host.
+// Whether a general-gap solve's folds return the strict folds' bits in any
+// order: similarities and costs finite (sums cannot overflow) or, for
+// similarities, the worst value, and no candidate -0 (a sum is -0 only where
+// both terms are: no similarity is, and not both a border cell and a cost).
+// Device-resident dense similarities are not read here: false.
+bool wsb_any_order(const pa_solver &s, const Input &in, const Job &job) {
+    auto finite = [](float x) { return std::fabs(x) <= 1e30f; };
+    auto neg0 = [](float x) { return x == 0.0f && std::signbit(x); };
+    bool cost0 = false, border0 = false;
+    for (const std::vector<float> *w : {&s.ws_sgn, &s.wt_sgn})
+        for (size_t k = 1; k < w->size(); k++) {
+            if (!finite((*w)[k])) return false;
+            cost0 = cost0 || neg0((*w)[k]);
+        }
+    for (const std::vector<float> *b : {&s.border_s, &s.border_t})
+        for (size_t k = 0; k < b->size(); k++) {
+            if (!finite((*b)[k])) return false;
+            border0 = border0 || (k > 0 && neg0((*b)[k]));
+        }
+    if (cost0 && border0) return false;
+    if (job.form == F_BINARY) return finite(in.eq) && finite(in.ne) && !neg0(in.eq) && !neg0(in.ne);
+    const float w = worst(s.opt.dir);
+    auto good = [&](float x) { return (finite(x) && !neg0(x)) || x == w; };
+    if (job.form == F_DENSE)
+        return !in.on_device && std::all_of(in.dense, in.dense + in.dense_elems, good);
+    return std::all_of(in.table.begin(), in.table.end(), good);
+}
+
+int32_t wsb_blocks(int32_t n) { return (n + WSB_TILE - 1) / WSB_TILE; }
+
+// The block launches of problems sorted by their number of anti-diagonals.
+WsbPlan wsb_plan(const std::vector<Prob> &probs, int cus) {
+    WsbPlan plan{};
+    plan.n = int64_t(probs.size());
+    int64_t widest = 0, problems = 0;
+    int32_t longest = 0;
+    for (const Prob &pr : probs) {
+        const int32_t bs = wsb_blocks(pr.len_s), bt = wsb_blocks(pr.len_t);
+        if (!bs || !bt) break;
+        problems++;
+        widest += std::min(bs, bt);
+        longest = std::max(longest, bs + bt);
+        plan.reach = std::max(plan.reach, std::max(bs, bt) - 2);
+    }
+    // Carried sums cost a load and a store of 256 sums per pair of blocks and
+    // pay where an anti-diagonal's blocks are few and have many blocks before
+    // them: one pair of 75 x 63 blocks 3.5 -> 1.6 ms.  Four problems to a
+    // workgroup fold without idle lanes where there are enough of them.
+    plan.carry = longest >= 24 && widest < int64_t(cus) * 8;
+    plan.across = !plan.carry && problems >= 16;
+    auto on_diag = [&](const Prob &pr, int32_t d) {
+        const int32_t bs = wsb_blocks(pr.len_s), bt = wsb_blocks(pr.len_t);
+        return !bs || !bt || d < 0 ? 0 : std::max(0, std::min(d, bs - 1) - std::max(0, d - bt + 1) + 1);
+    };
+    for (int32_t d = 0;; d++) {
+        WsbPlan::Diag g{};
+        int64_t total = 0;
+        for (const Prob &pr : probs) {
+            const int32_t n = on_diag(pr, d);
+            if (!n) break;
+            g.problems++;
+            g.groups = std::max(g.groups, plan.across ? n : (n + 3) / 4);
+            g.sources = std::max(g.sources, (on_diag(pr, d - 1) + 3) / 4);
+            total += n;
+        }
+        if (!g.problems) return plan;
+        g.waves = 1;
+        if (plan.carry) g.waves = 2;
+        else  // four waves per SIMD where there is that much to fold
+            while (g.waves < 8 && g.waves < 2 * d && total / 4 * g.waves < 16 * int64_t(cus)) g.waves *= 2;
+        plan.diags.push_back(g);
+    }
+}
+
+// General gap costs (Waterman-Smith-Beyer), no strip schedule.  Scores and
+// one optimal path are computed in blocks where the folds may take any order;
+// otherwise one workgroup per problem leaves D, S and the traceback codes of
+// every cell in device memory, which all-optimal enumeration and Solution
+// matrices read on the host.
 void run_wsb(pa_solver &s, const Input &in, const Job &job, std::unique_ptr<pa_result> *result,
              float *scores_device) {
     const pa_options &o = s.opt;
     const int64_t n = in.n;
     if (!s.gen_ready) fail(PA_EINVAL, "general gap costs were not given to the solver");
     hipStream_t st = s.stream;
+    const bool blocks = job.tr != TR_ALL && !in.matrices && wsb_any_order(s, in, job);
     std::vector<Prob> probs(static_cast<size_t>(n));
     int64_t words = 0;
     double cells = 0;
@@ -910,12 +986,35 @@ void run_wsb(pa_solver &s, const Input &in, const Job &job, std::unique_ptr<pa_r
             pr.off_s = in.off_s[k];
             pr.off_t = in.off_t[k];
         }
-        pr.dv_off = words;
-        words += int64_t(WSB_PLANES) * pr.len_s * pr.len_t;
         cells += double(pr.len_s) * double(pr.len_t);
+    }
+    WsbPlan plan{};
+    if (blocks) {
+        auto shape = [](const Prob &pr) {
+            const int32_t bs = wsb_blocks(pr.len_s), bt = wsb_blocks(pr.len_t);
+            return bs && bt ? std::make_pair(bs + bt, bs) : std::make_pair(0, 0);
+        };
+        std::stable_sort(probs.begin(), probs.end(),
+                         [&](const Prob &x, const Prob &y) { return shape(x) > shape(y); });
+        plan = wsb_plan(probs, s.cus);
+    }
+    for (Prob &pr : probs) {
+        const int64_t nb = int64_t(wsb_blocks(pr.len_s)) * wsb_blocks(pr.len_t);
+        pr.dv_off = words;
+        words += int64_t(blocks ? 2 : WSB_PLANES) * pr.len_s * pr.len_t;
+        if (blocks && job.loc == LOC_LOCAL) {
+            pr.rb_off = words;
+            words += 2 * nb;
+        }
+        if (plan.carry) {
+            pr.tb_off = words;
+            words += 2 * WSB_TILE * WSB_TILE * nb;
+        }
     }
     upload(st, s.b_probs, probs.data(), probs.size());
     s.last_plan.uploaded = false;  // b_probs now holds these descriptors
+    s.b_ws.ensure((s.ws_sgn.size() + WSB_TILE) * 4);
+    s.b_wt.ensure((s.wt_sgn.size() + WSB_TILE) * 4);
     upload(st, s.b_ws, s.ws_sgn.data(), s.ws_sgn.size());
     upload(st, s.b_wt, s.wt_sgn.data(), s.wt_sgn.size());
     const void *codes_s = nullptr, *codes_t = nullptr;
@@ -970,14 +1069,17 @@ void run_wsb(pa_solver &s, const Input &in, const Job &job, std::unique_ptr<pa_r
     // 1024 (one thread per cell of the longest anti-diagonal) for more loads
     // in flight per problem
     int threads = 256;
-    if (n < s.cus) {
+    if (!blocks && n < s.cus) {
         int64_t diag = 0;
         for (int64_t k = 0; k < n; k++) diag = std::max<int64_t>(diag, std::min(in.len_s[k], in.len_t[k]));
         threads = int(std::min<int64_t>(1024, std::max<int64_t>(256, (diag + 63) / 64 * 64)));
     }
     HIPCHK(hipEventRecord(s.ev0, st));
-    const hipError_t le = launch_wsb(job.loc, job.dir, job.form, a, n, s.b_ws.as<float>(), s.b_wt.as<float>(),
-                                     path, path_off, path_len, threads, st);
+    const hipError_t le =
+        blocks ? launch_wsb_blocks(job.loc, job.dir, job.form, a, plan, s.b_ws.as<float>(), s.b_wt.as<float>(), path,
+                                   path_off, path_len, st)
+               : launch_wsb(job.loc, job.dir, job.form, a, n, s.b_ws.as<float>(), s.b_wt.as<float>(), path, path_off,
+                            path_len, threads, st);
     if (le != hipSuccess) {
         std::ostringstream m;
         m << "kernel launch failed (general gap costs, loc " << job.loc << " dir " << job.dir << " form "
@@ -985,7 +1087,7 @@ void run_wsb(pa_solver &s, const Input &in, const Job &job, std::unique_ptr<pa_r
         fail(PA_EHIP, m.str());
     }
     HIPCHK(hipEventRecord(s.ev1, st));
-    s.last_launches = 1;
+    s.last_launches = blocks ? int(plan.diags.size()) : 1;
     s.last_cells = cells;
     s.last_groups = 0;
     s.last_band = 0;

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 namespace pa {
 
 enum { LOC_LOCAL = 0, LOC_GLOBAL = 1, LOC_SEMI = 2 };
@@ -266,6 +268,30 @@ constexpr int WSB_PLANES = 4;
 hipError_t launch_wsb(int loc, int dir, int form, const KArgs &args, int64_t n, const float *ws, const float *wt,
                       int32_t *path, const int64_t *path_off, int32_t *path_len, int threads,
                       hipStream_t stream);
+// The same in blocks of WSB_TILE x WSB_TILE cells (pa_wsb.hip), one launch
+// per block anti-diagonal: scores and one optimal path of values whose folds
+// may take any order.  At dvals + dv_off it writes two ls x lt planes, D and
+// D transposed, for local problems at dvals + rb_off two words per block (its
+// best cell), and with `carry` at dvals + tb_off two blocks of sums per block.
+// The problems are sorted by their number of block anti-diagonals, most first;
+// ws / wt have WSB_TILE readable floats past their ends.
+constexpr int WSB_TILE = 16;
+struct WsbPlan {
+    int64_t n;     // problems, empty ones included
+    bool across;   // a workgroup's four blocks: of four problems (else neighbours of one)
+    bool carry;    // every block's values are pushed on once (else later blocks fold all before them)
+    int32_t reach; // carry: blocks that a block is pushed to, at most, per direction
+    struct Diag {
+        int32_t problems;  // with this anti-diagonal
+        int32_t groups;    // workgroups per problem (four problems), at most
+        int32_t waves;     // per workgroup, sharing the folds of its four blocks
+        int32_t sources;   // carry: groups of four blocks of the anti-diagonal before, at most, per problem
+    };
+    std::vector<Diag> diags;
+};
+hipError_t launch_wsb_blocks(int loc, int dir, int form, const KArgs &args, const WsbPlan &plan, const float *ws,
+                             const float *wt, int32_t *path, const int64_t *path_off, int32_t *path_len,
+                             hipStream_t stream);
 bool supported_R(int form, int tr, bool fastmax, int R);
 // The allocation-free entry point's device memory: a file-scope device array
 // of NOALLOC_SCRATCH_BYTES per GPU.  noalloc_scratch gives the current
