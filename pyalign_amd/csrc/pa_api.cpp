@@ -144,6 +144,7 @@ struct Plan {
     std::vector<int32_t> band_probs;   // their indices in probs (long-mode problems first)
     int32_t n_long = 0;                // long-mode problems (pa_long_kernel): band_probs[0 .. n_long)
     int32_t long_bands = 0;            // their bands (workgroup tickets)
+    std::vector<int32_t> band_words;   // device copy: band_probs, then (problem, band) of every ticket
     int64_t xbuf_begin = 0, xbuf_end = 0;  // float2 range of the row buffer holding their tagged hand-offs
 };
 
@@ -426,10 +427,13 @@ bool choose_layout(int64_t ls, int64_t lt, const std::vector<int> &Rs, double ca
     int bL = 64, bR = Rs.back();
     double fb_serial = 1e300, fb_cost = 1e300;
     int fL = 64, fR = Rs.back();
-    for (int L = 1; L <= 64; L <<= 1) {
-        for (int R : Rs) {
-            const int64_t rps = int64_t(L) * R;
-            const int64_t nst = (ls + rps - 1) / rps;
+    int32_t lanes[16];  // lanes of R rows (one division per strip height, not per layout)
+    for (size_t q = 0; q < Rs.size(); q++) lanes[q] = int32_t((ls + Rs[q] - 1) / Rs[q]);
+    for (int lg = 0; lg <= 6; lg++) {
+        const int L = 1 << lg;
+        for (size_t q = 0; q < Rs.size(); q++) {
+            const int R = Rs[q];
+            const int32_t nst = (lanes[q] + L - 1) >> lg;
             const double serial = double(nst) * double(lt + L - 1) * (STEP_OVERHEAD + R);
             const double cost = serial * L;
             if (serial < fb_serial || (serial == fb_serial && cost < fb_cost)) {
@@ -476,7 +480,8 @@ double band_serial(int64_t ls, int64_t lt, int R, int *nst_out) {
 
 struct Job {
     int loc, dir, gap, form, tr;
-    bool fast;
+    bool fold_max;  // max / min folds keep the strict folds' bits (folds_max)
+    bool fast;      // the score kernel
 };
 
 // ckpt[k] != 0: problem k keeps no traceback (a checkpointed forward): one
@@ -487,34 +492,46 @@ struct Job {
 // long_dw phases of LONG_T steps apart within a workgroup (rows handed down
 // through LDS) and a little more between workgroups, so the serial time is
 // (len_t + 63 + (strips - 1) * long_dw * LONG_T * ~1.25) steps of one row.
-// A step of one row costs about 50 ns (measured), three cell units of the
-// general kernel (R = 8: a 12-unit step in about 200 ns) and four of the
-// fast kernel's cheaper cells.
-double long_serial(int64_t ls, int64_t lt, int form, bool fast, int *nst_out) {
+// Measured per step of one row: 63 ns score only, 100 ns with traceback codes,
+// against about 14 ns per cell unit of the score kernel, 50 ns per unit of the
+// general kernel with codes and 20 ns without.
+double long_unit(const Job &job) { return job.fast ? 4.5 : (job.tr == TR_ONE ? 2.0 : 3.0); }
+
+double long_serial(int64_t ls, int64_t lt, const Job &job, int *nst_out) {
     const int64_t nst = (ls + WAVE * LONG_R - 1) / (WAVE * LONG_R);
     *nst_out = int(nst);
-    return double(lt + WAVE - 1 + double(nst - 1) * long_dw(form) * LONG_T * 1.25) * (fast ? 4.0 : 3.0);
+    return double(lt + WAVE - 1 + double(nst - 1) * long_dw(job.form) * LONG_T * 1.25) * long_unit(job);
+}
+
+// a workgroup's time for one band of a problem: its last wave starts
+// LONG_WAVES - 1 hand-off distances after the first
+double long_band(int64_t lt, const Job &job) {
+    return double(lt + WAVE - 1 + ((LONG_WAVES - 1) * long_dw(job.form) + 2) * LONG_T) * long_unit(job);
 }
 
 Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, int simds,
                const uint8_t *ckpt = nullptr, bool allow_band = true, bool allow_long = true) {
     std::vector<int> Rs;
     if (job.fast) {
-        Rs.assign(std::begin(FAST_RS), std::end(FAST_RS));
+        if (job.form == F_BINARY) Rs.assign(std::begin(FAST_RS_BINARY), std::end(FAST_RS_BINARY));
+        else if (job.loc == LOC_LOCAL && job.dir == DIR_MAX) Rs.assign(std::begin(FAST_RS), std::end(FAST_RS));
+        else Rs.assign(std::begin(FAST_RS_TABLE), std::end(FAST_RS_TABLE));
     } else {
-        for (int R : {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32})
-            if (supported_R(job.form, job.tr, job.fast, R)) Rs.push_back(R);
+        for (int R : {4, 8, 16, 32})
+            if (supported_R(job.form, job.tr, R)) Rs.push_back(R);
     }
     // total wavefront time at the cheapest layouts (no cap) sets the cap:
     // an eighth of a SIMD's share of the work for the fast kernel, a
     // sixteenth for the general kernel (both measured best)
+    // (of a large bag every few problems stand for all)
+    const int64_t stride = std::max<int64_t>(1, n / 4096);
     double total = 0.0;
-    for (int64_t k = 0; k < n; k++) {
+    for (int64_t k = 0; k < n; k += stride) {
         if (ls[k] <= 0 || lt[k] <= 0) continue;
         int L, R;
         double cost = 0.0;
         choose_layout(ls[k], lt[k], Rs, 1e300, L, R, &cost);
-        total += cost / 64.0;
+        total += cost / 64.0 * double(std::min(stride, n - k));
     }
 #ifndef PA_CAP_DIV
 #define PA_CAP_DIV 8.0
@@ -522,7 +539,46 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
 #ifndef PA_CAP_DIV_GENERAL
 #define PA_CAP_DIV_GENERAL 16.0
 #endif
-    const double cap = std::max(256.0, total / (double(simds) * (job.fast ? PA_CAP_DIV : PA_CAP_DIV_GENERAL)));
+    double cap = std::max(256.0, total / (double(simds) * (job.fast ? PA_CAP_DIV : PA_CAP_DIV_GENERAL)));
+    // With few problems per SIMD that cap lies below every layout's serial
+    // time, and the layouts of least serial time waste most of their lanes:
+    // the cap is doubled while the estimated time (the larger of the work per
+    // SIMD and the longest problem, and half the other; the longest alone where
+    // there is no more than a wavefront per SIMD) falls by a tenth in one or two
+    // doublings.  On a sample of the problems.  16,384 semiglobal pairs of
+    // 125 x 300: kernel 0.50 -> 0.29 ms; 1,039 DTW training pairs of up to 2,499
+    // (a few more than SIMDs): 11.5 -> 9.2 ms.
+    {
+        const int64_t every = std::max<int64_t>(1, n / 256);
+        double work = 0.0, longest = 0.0, waves = 0.0;
+        auto estimate = [&](double c) {
+            work = longest = waves = 0.0;
+            for (int64_t k = 0; k < n; k += every) {
+                if (ls[k] <= 0 || lt[k] <= 0) continue;
+                int L, R;
+                double cost = 0.0, serial = 0.0;
+                choose_layout(ls[k], lt[k], Rs, c, L, R, &cost, &serial);
+                work += cost / 64.0 * double(every) / simds;
+                waves += L / 64.0 * double(every);
+                longest = std::max(longest, serial);
+            }
+            if (waves <= simds) return longest;
+            return std::max(work, longest) + 0.5 * std::min(work, longest);
+        };
+        double best = estimate(cap), c = cap;
+        if (waves > simds && work > 0.25 * longest)
+            for (int missed = 0; missed < 2;) {
+                c *= 2.0;
+                const double t = estimate(c);
+                if (t < 0.9 * best) {
+                    best = t;
+                    cap = c;
+                    missed = 0;
+                } else {
+                    missed++;
+                }
+            }
+    }
     // band mode only for a problem that would otherwise be the critical path
     // (serial time above the balanced per-SIMD total); its strips run in the
     // general kernel, several times slower per cell than the fast one
@@ -530,7 +586,7 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
 #define PA_BAND_CRIT 4.0
 #endif
     const double crit = PA_BAND_CRIT * cap;
-    const double band_penalty = job.fast ? 3.0 : 1.0;
+    const double band_penalty = job.fast && job.form == F_TABLE && job.loc == LOC_LOCAL && job.dir == DIR_MAX ? 3.0 : 1.0;
 
     struct Item {
         int64_t k;
@@ -539,16 +595,40 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
         double band;  // > 0: band mode, its serial time
         bool ckpt;    // a checkpointed problem (strip rows kept, no traceback)
     };
-    const bool band_ok = allow_band && job.tr != TR_ALL && supported_R(job.form, job.tr, false, BAND_R);
+    const bool band_ok = allow_band && job.tr != TR_ALL && supported_R(job.form, job.tr, BAND_R);
     const bool long_ok = allow_band && allow_long && !std::getenv("PYALIGN_AMD_NO_LONG_MODE") &&
                          long_supported(job.gap, job.form, job.tr);
     std::vector<Item> items(static_cast<size_t>(n));
     std::vector<Item> bands, ckpts, longs;
+    struct Cand {
+        int64_t k;
+        double serial, cost, long_serial, long_cost;
+        int nst;
+    };
+    std::vector<Cand> cands;  // problems the long mode could take
+    struct Layout {  // of the shapes met last (bags of short problems repeat theirs)
+        int32_t ls = 0, lt = 0, L = 0, R = 0;
+        double cost = 0.0, serial = 0.0;
+        bool fit = false;
+    };
+    std::vector<Layout> memo(n >= 4096 ? 1024 : 1);
     for (int64_t k = 0; k < n; k++) {
         int L = 64, R = Rs.back();
-        double serial = 0.0;
+        double serial = 0.0, cost = 0.0;
         bool fit = true;
-        if (ls[k] > 0 && lt[k] > 0) fit = choose_layout(ls[k], lt[k], Rs, cap, L, R, nullptr, &serial);
+        if (ls[k] > 0 && lt[k] > 0) {
+            Layout &m = memo[(size_t(ls[k]) * 31 + size_t(lt[k])) % memo.size()];
+            if (m.ls != ls[k] || m.lt != lt[k]) {
+                m.ls = ls[k];
+                m.lt = lt[k];
+                m.fit = choose_layout(ls[k], lt[k], Rs, cap, m.L, m.R, &m.cost, &m.serial);
+            }
+            L = m.L;
+            R = m.R;
+            cost = m.cost;
+            serial = m.serial;
+            fit = m.fit;
+        }
         else { L = 1; R = Rs.front(); }
         const int64_t rps = int64_t(L) * R;
         const int nst = ls[k] > 0 && lt[k] > 0 ? int((ls[k] + rps - 1) / rps) : 0;
@@ -561,18 +641,14 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
             items[size_t(k)] = Item{k, 0, 0, 0, 0, 0.0, false};
             continue;
         }
-        // where the long mode serves the job it replaces band mode (whose
-        // strips hand rows down through published column counts, several
-        // times slower per step than the long mode's LDS rings)
         if (!fit && long_ok && serial > crit) {
             int nl = 0;
-            const double sl = long_serial(ls[k], lt[k], job.form, job.fast, &nl);
+            const double sl = long_serial(ls[k], lt[k], job, &nl);
             // (at least one strip per compute wave of a workgroup: shorter
             // problems leave its waves idle)
             if (nl >= LONG_WAVES && sl < serial) {
-                longs.push_back(Item{k, WAVE, LONG_R, nl, lt[k], sl, false});
-                items[size_t(k)] = Item{k, 0, 0, 0, 0, 0.0, false};
-                continue;
+                const double lc = double((nl + LONG_WAVES - 1) / LONG_WAVES) * long_band(lt[k], job);
+                cands.push_back(Cand{k, serial, cost / 64.0, sl, lc, nl});
             }
         }
         if (!fit && band_ok && !long_ok && serial > crit) {
@@ -587,16 +663,57 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
         }
         items[size_t(k)] = Item{k, L, R, nst, lt[k], 0.0, false};
     }
+    // Where the long mode serves the job it replaces band mode (whose strips
+    // hand rows down through published column counts, several times slower per
+    // step than the long mode's LDS rings).  A workgroup of it fills a CU and
+    // its waves wait about half their time, so of the problems it could take it
+    // gets the longest ones only while that shortens the whole: both launches
+    // last as long as their longest problem or their work spread over the GPU
+    // (SIMDs; a band per CU), one after the other.  (16,384 global pairs of 50
+    // to 1,000, score only: every problem above a quarter of a SIMD's share
+    // 8.6 ms, none 0.65 ms.)
+    if (!cands.empty()) {
+        std::stable_sort(cands.begin(), cands.end(), [](const Cand &a, const Cand &b) { return a.serial > b.serial; });
+        double rest = total, long_max = 0.0, long_sum = 0.0;
+        double best = std::max(cands[0].serial, total / simds);
+        size_t take = 0;
+        for (size_t q = 0; q < cands.size(); q++) {
+            rest -= cands[q].cost;
+            long_max = std::max(long_max, cands[q].long_serial);
+            long_sum += cands[q].long_cost;
+            const double next = q + 1 < cands.size() ? cands[q + 1].serial : (int64_t(q) + 1 < n ? crit : 0.0);
+            const double t = std::max(long_max, long_sum / (double(simds) / 4.0)) +
+                             std::max(next, std::max(rest, 0.0) / simds);
+            if (t < best) {
+                best = t;
+                take = q + 1;
+            }
+        }
+        for (size_t q = 0; q < take; q++) {
+            const Cand &c = cands[q];
+            longs.push_back(Item{c.k, WAVE, LONG_R, c.nst, lt[c.k], c.long_serial, false});
+            items[size_t(c.k)] = Item{c.k, 0, 0, 0, 0, 0.0, false};
+        }
+    }
     if (!bands.empty() || !ckpts.empty() || !longs.empty())
         items.erase(std::remove_if(items.begin(), items.end(), [](const Item &it) { return it.L == 0; }),
                     items.end());
-    // group identical layouts with similar shape: sort by R, L, strips, len_t
-    std::stable_sort(items.begin(), items.end(), [](const Item &a, const Item &b) {
-        if (a.R != b.R) return a.R < b.R;
-        if (a.L != b.L) return a.L < b.L;
-        if (a.nst != b.nst) return a.nst > b.nst;
-        return a.lt > b.lt;
-    });
+    // group identical layouts with similar shape: sort by R, L, strips (most
+    // first), len_t (longest first), one key per problem
+    {
+        std::vector<std::pair<uint64_t, uint32_t>> order(items.size());
+        for (size_t q = 0; q < items.size(); q++) {
+            const Item &it = items[q];
+            const uint64_t nst = uint64_t(0x3fffff - std::min(it.nst, 0x3fffff));
+            order[q] = {uint64_t(it.R) << 57 | uint64_t(ilog2(it.L)) << 54 | nst << 32 |
+                            uint64_t(0x7fffffff - std::min<int64_t>(it.lt, 0x7fffffff)),
+                        uint32_t(q)};
+        }
+        std::sort(order.begin(), order.end());
+        std::vector<Item> sorted(items.size());
+        for (size_t q = 0; q < items.size(); q++) sorted[q] = items[order[q].second];
+        items.swap(sorted);
+    }
     Plan plan;
     plan.probs.reserve(static_cast<size_t>(n));
     struct GroupR {
@@ -614,7 +731,13 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
         g.lgL = ilog2(L);
         g.strip = -1;
         int cnt = 0;
+        double most = 0.0;  // the members' longest serial time; a group ends before it runs much longer than that
         while (p < items.size() && cnt < per && items[p].L == L && items[p].R == R) {
+            const double own = double(items[p].nst) * double(items[p].lt + L - 1);
+            const double together = double(std::max<int32_t>(g.max_nst, items[p].nst)) *
+                                    double(std::max<int64_t>(g.max_lt, items[p].lt) + L - 1);
+            most = std::max(most, own);
+            if (cnt && together > 1.25 * most) break;
             Prob pr{};
             pr.out = int32_t(items[p].k);
             pr.L = L;
@@ -670,6 +793,23 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
         plan.n_long++;
         plan.probs.push_back(pr);
     }
+    // The tickets' order: the longest way still to go first (the bands below
+    // one start about long_dw phases per strip after it), so that a band comes
+    // after those above it and, with more bands than workgroups, problems
+    // advance side by side instead of waiting for their own band above.
+    struct Ticket {
+        int32_t prob, band;
+        double rest;
+    };
+    std::vector<Ticket> tickets;
+    tickets.reserve(size_t(plan.long_bands));
+    for (size_t q = 0; q < longs.size(); q++) {
+        const int32_t nb = (longs[q].nst + LONG_WAVES - 1) / LONG_WAVES;
+        for (int32_t b = 0; b < nb; b++)
+            tickets.push_back(Ticket{plan.band_probs[q], b,
+                                     double(longs[q].lt) + double(nb - b) * LONG_WAVES * long_dw(job.form) * LONG_T * 1.25});
+    }
+    std::stable_sort(tickets.begin(), tickets.end(), [](const Ticket &a, const Ticket &b) { return a.rest > b.rest; });
     // band-mode problems: one group per strip, strips in order, run by the
     // general kernel (its launch goes first: it holds the longest problems)
     std::stable_sort(bands.begin(), bands.end(), [](const Item &a, const Item &b) { return a.band > b.band; });
@@ -705,6 +845,11 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
         if (a.R != b.R) return a.R > b.R;
         return a.g.cost > b.g.cost;
     });
+    plan.band_words = plan.band_probs;
+    for (const Ticket &t : tickets) {
+        plan.band_words.push_back(t.prob);
+        plan.band_words.push_back(t.band);
+    }
     size_t q = 0;
     while (q < gs.size()) {
         const int R = gs[q].R;
@@ -808,6 +953,31 @@ struct Input {
     // (F_TABLE_G) instead of staged in LDS with uint8 codes
     bool table_g = false;
 };
+
+// Whether max / min folds (and traceback codes from equality tests) keep the
+// strict folds' bits in alignments over a table or binary symbols:
+// similarities finite (or the pad's worst value) and never -0, and, for
+// maximising global problems, gap costs above zero (borders below -0), so that
+// no candidate is -0 or NaN.
+bool folds_max(const pa_solver &s, const Input &in, const Job &job) {
+    if (job.gap != GAP_LIN && job.gap != GAP_AFF) return false;
+    auto exact = [](float x) { return std::isfinite(x) && !(x == 0.0f && std::signbit(x)); };
+    if (job.loc == LOC_GLOBAL && job.dir == DIR_MAX && !(s.go_s < 0.0f && s.go_t < 0.0f)) return false;
+    if (job.form == F_BINARY) return exact(in.eq) && exact(in.ne);
+    if (job.form != F_TABLE) return false;
+    const float w = worst(s.opt.dir);
+    return std::all_of(in.table.begin(), in.table.end(), [&](float x) { return exact(x) || x == w; });
+}
+
+// Whether the score kernel serves a job.  The local maximum over a table needs
+// no NaN only; a local binary problem's padded rows score ne, which must not
+// lift them above the optimum.
+bool score_kernel(const Input &in, const Job &job) {
+    if (job.tr != TR_SCORE || (job.gap != GAP_LIN && job.gap != GAP_AFF)) return false;
+    if (job.form == F_TABLE) return job.fold_max || (job.loc == LOC_LOCAL && job.dir == DIR_MAX && in.nan_free);
+    if (job.form != F_BINARY || !job.fold_max) return false;
+    return job.loc != LOC_LOCAL || (job.dir == DIR_MAX ? in.ne <= 0.0f : in.ne >= 0.0f);
+}
 
 int goal_to_tr(int goal) { return goal == PA_GOAL_SCORE ? TR_SCORE : (goal == PA_GOAL_ONE ? TR_ONE : TR_ALL); }
 
@@ -1135,11 +1305,8 @@ void run_wsb(pa_solver &s, const Input &in, const Job &job, std::unique_ptr<pa_r
     *result = std::move(r);
 }
 
-bool is_long(const Plan &pl, const Prob &pr) {
-    for (int32_t q = 0; q < pl.n_long; q++)
-        if (&pl.probs[size_t(pl.band_probs[size_t(q)])] == &pr) return true;
-    return false;
-}
+// (only long-mode problems hold one row per lane)
+bool is_long(const Prob &pr) { return pr.R == LONG_R && pr.band >= 0; }
 
 // A plan's problems get their lengths and offsets: payload, traceback
 // words, strip-boundary row buffer and cell values.
@@ -1165,14 +1332,14 @@ void place_plan(Plan &pl, const Input &in, int bits, bool keep_vals, int val_lay
             // rows (the walk loads them four words at a time)
             if (pr.L == WAVE && pr.R == 1) pl.tb_words = (pl.tb_words + 3) & ~int64_t(3);
             pr.tb_off = pl.tb_words;
-            if (is_long(pl, pr)) {  // codes packed along the steps
+            if (is_long(pr)) {  // codes packed along the steps
                 pr.pack = long_pack(bits);
                 pl.tb_words += nst * long_strip_words(pr.len_t + WAVE - 1, bits) * WAVE;
             } else {
                 pl.tb_words += nst * (pr.len_t + pr.L - 1) * pr.L * ((bits * pr.R + 31) / 32);
             }
         }
-        if (nst > 1 && !is_long(pl, pr)) {
+        if (nst > 1 && !is_long(pr)) {
             pr.rb_off = pl.rowbuf;
             pl.rowbuf += pr.band >= 0 ? (nst - 1) * int64_t(pr.len_t) : int64_t(pr.len_t);
         }
@@ -1226,11 +1393,12 @@ void build_launches(pa_solver &s, const Job &job, const Input &in, const Plan &p
         spec.R = R;
         spec.fastmax = fastmax;
         spec.lds_bytes = job.form == F_TABLE ? size_t(in.K1) * in.K1 * 4 : 0;
+        spec.var = job.tr == TR_SCORE ? VAR_PLAIN : a.dvals ? VAR_VALUES : job.fold_max ? VAR_MAX : VAR_PLAIN;
         if (drows && R == DROWS_WIN) {
             spec.form = F_DROWS;
             spec.lds_bytes = DROWS_LDS;
         }
-        if (fastmax && R == 0 && in.K1 >= 2) {
+        if (fastmax && job.form == F_TABLE && in.K1 >= 2) {
             const size_t pair_bytes = size_t(in.K1) * in.K1 * (in.K1 - 1) * 8;
             if (pair_bytes <= PAIR_LDS_MAX && !s.no_pair) {
                 spec.pair = 1;
@@ -1238,7 +1406,7 @@ void build_launches(pa_solver &s, const Job &job, const Input &in, const Plan &p
             }
         }
         const std::vector<int> okey = {spec.loc, spec.dir, spec.gap, spec.form, spec.tr, spec.R,
-                                       int(spec.fastmax), int(spec.lds_bytes), spec.pair, in.dim};
+                                       int(spec.fastmax), int(spec.lds_bytes), spec.pair, in.dim, spec.var};
         int waves_per_cu = 0;
         for (auto &e : s.occ_cache)
             if (e.first == okey) waves_per_cu = e.second;
@@ -1304,8 +1472,8 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
     }
     const int val_layers = in.matrices && job.gap == GAP_AFF ? 3 : 1;
     const bool keep_vals = in.matrices || (job.tr == TR_ALL && job.loc == LOC_LOCAL);
-    job.fast = job.form == F_TABLE && job.tr == TR_SCORE && job.loc == LOC_LOCAL && job.dir == DIR_MAX &&
-               o.gap != GAP_DTW && in.nan_free;
+    job.fold_max = folds_max(s, in, job);
+    job.fast = score_kernel(in, job);
 
     hipStream_t st = s.stream;
     // ---- schedule (reused while lengths, offsets and job repeat) ------------
@@ -1365,7 +1533,7 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
     if (!pc.uploaded) {
         const Plan &pl = pc.plan;
         const size_t nb[3] = {pl.probs.size() * sizeof(Prob), pl.groups.size() * sizeof(Group),
-                              pl.band_probs.size() * sizeof(int32_t)};
+                              pl.band_words.size() * sizeof(int32_t)};
         const size_t al = 256, total = (nb[0] + al) + (nb[1] + al) + (nb[2] + al);
         if (s.stage_pending) HIPCHK(hipEventSynchronize(s.stage_ev));
         s.stage_pending = false;
@@ -1376,7 +1544,7 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
             HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&s.stage), total + total / 4, hipHostMallocDefault));
             s.stage_cap = total + total / 4;
         }
-        const void *src[3] = {pl.probs.data(), pl.groups.data(), pl.band_probs.data()};
+        const void *src[3] = {pl.probs.data(), pl.groups.data(), pl.band_words.data()};
         DevBuf *dst[3] = {&s.b_probs, &s.b_groups, &s.b_band_probs};
         size_t at = 0;
         for (int q = 0; q < 3; q++) {
@@ -1467,31 +1635,8 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
     const int n_band = int(plan.band_probs.size());
     LongArgs la{};
     int long_grid = 0;
-    // the long kernel folds cells with max / min (and takes traceback codes
-    // from equality tests) where that keeps the strict fold's bits:
-    // similarities finite (or the pad's worst value) and never -0, and, for
-    // maximising global problems, gap costs above zero (borders below -0), so
-    // that no candidate is -0 or NaN
-    bool fold_max = false;
     if (plan.n_long > 0) {
-        auto exact = [](float x) { return std::isfinite(x) && !(x == 0.0f && std::signbit(x)); };
-        bool good = true;
-        if (job.form == F_BINARY) {
-            good = exact(in.eq) && exact(in.ne);
-        } else {
-            const float w = worst(o.dir);
-            for (float x : in.table)
-                if (!exact(x) && x != w) {
-                    good = false;
-                    break;
-                }
-        }
-        if (job.loc == LOC_GLOBAL && job.dir == DIR_MAX && !(s.go_s < 0.0f && s.go_t < 0.0f)) good = false;
-        fold_max = good;
-    }
-    if (plan.n_long > 0) {
-        la.idx = s.b_band_probs.as<int32_t>();
-        la.n = plan.n_long;
+        la.order = s.b_band_probs.as<int32_t>() + n_band;
         la.total_bands = plan.long_bands;
         la.ticket = s.b_queue.as<uint32_t>() + plan.launches.size();
         long_grid = std::max(1, std::min(plan.long_bands, s.cus));
@@ -1510,7 +1655,7 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
             e = launch_zero_u32(reinterpret_cast<uint32_t *>(s.b_rowbuf.as<float2>() + plan.xbuf_begin),
                                 2 * (plan.xbuf_end - plan.xbuf_begin), st);
         if (e == hipSuccess && plan.n_long > 0)
-            e = launch_long(job.loc, job.dir, job.gap, job.form, job.tr, fold_max, a, la, long_grid, st);
+            e = launch_long(job.loc, job.dir, job.gap, job.form, job.tr, job.fold_max, a, la, long_grid, st);
         for (size_t q = 0; q < specs.size() && e == hipSuccess; q++) e = launch_solve(specs[q], largs[q], st);
         if (e == hipSuccess && n_band > 0)
             e = launch_band_combine(job.loc, job.dir, job.tr, s.b_probs.as<Prob>(), s.b_band_probs.as<int32_t>(),
@@ -1525,7 +1670,7 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
     const int64_t extra[10] = {int64_t(plan.launches.size()), plan.band_slots, n_band,
                                int64_t(reinterpret_cast<intptr_t>(scores)), int64_t(reinterpret_cast<intptr_t>(seeds)),
                                int64_t(job.loc * 100 + job.dir * 10 + job.tr), plan.n_long, plan.long_bands,
-                               (plan.xbuf_end - plan.xbuf_begin) * 2 + int64_t(fold_max),
+                               (plan.xbuf_end - plan.xbuf_begin) * 2 + int64_t(job.fold_max),
                                int64_t(reinterpret_cast<intptr_t>(s.b_band_probs.p))};
     gkey.append(reinterpret_cast<const char *>(extra), sizeof(extra));
 
@@ -2182,8 +2327,8 @@ int pa_solve_ragged_scores_noalloc(pa_solver *s, const pa_ragged *batch, int32_t
         if (o.type == PA_TYPE_DTW && job.form != F_DENSE && job.form != F_SERIES)
             fail(PA_EINVAL, "DTW solvers take dense costs or series");
         if (job.form == F_SERIES && (in.dim < 1 || in.dim > 4)) fail(PA_EINVAL, "series dimension must be 1..4");
-        job.fast = job.form == F_TABLE && job.loc == LOC_LOCAL && job.dir == DIR_MAX && o.gap != GAP_DTW &&
-                   in.nan_free;
+        job.fold_max = folds_max(*s, in, job);
+        job.fast = score_kernel(in, job);
 
         void *base = nullptr;
         int cus = 0;

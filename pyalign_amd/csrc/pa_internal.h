@@ -27,6 +27,10 @@ constexpr size_t DROWS_LDS = size_t(256) * DROWS_LANE_FLOATS * 4;
 // What the forward pass keeps: score only, one traceback direction per cell
 // (2 bits linear/DTW, 4 bits affine) or the full tie set (8 bits per cell).
 enum { TR_SCORE = 0, TR_ONE = 1, TR_ALL = 2 };
+// Builds of the general kernel that keeps a traceback: the usual one, one that
+// also stores cell values (KArgs::dvals), and alignments over a table or
+// binary symbols with max / min folds.
+enum { VAR_PLAIN = 0, VAR_VALUES = 1, VAR_MAX = 2 };
 
 constexpr int WAVE = 64;
 constexpr int MAX_LDS_TABLE = 129;  // K + 1 pad symbol
@@ -129,9 +133,8 @@ constexpr int64_t long_strip_words(int64_t steps_per_strip, int bits) {
 constexpr uint32_t LONG_SPIN_LIMIT = 1u << 20;  // re-reads before a wait gives up (about a second)
 
 struct LongArgs {
-    const int32_t *idx;    // the long problems' indices into KArgs::probs
-    int32_t n;             // long problems
-    int32_t total_bands;   // bands over all of them (tickets)
+    const int32_t *order;  // per ticket: the problem's index in KArgs::probs and the band
+    int32_t total_bands;   // bands over all problems (tickets)
     uint32_t *ticket;      // band ticket counter (zeroed before launch)
 };
 
@@ -174,20 +177,25 @@ struct KArgs {
 constexpr int SAFE_FLOATS = 16;
 constexpr int SINK_WORDS = 16;
 
-// R = 0 selects the kernel that serves every strip height in FAST_RS from
-// one queue (the group carries its R).
-#ifndef PA_FAST_RS_LIST
+// Strip heights of the score kernel, which serves them all from one queue (the
+// group carries its R): the local maximum over a table, other alignments over
+// a table, and binary symbols (local ones hold a score per row besides the
+// rows' symbols, which keeps R = 32 out of the registers).
 #define PA_FAST_RS_LIST 8, 10, 12, 14, 16, 20, 24, 28, 32
-#endif
+#define PA_FAST_RS_TABLE 4, 8, 12, 16, 20, 24
+#define PA_FAST_RS_BINARY 4, 8, 12, 16, 24
 constexpr int FAST_RS[] = {PA_FAST_RS_LIST};
+constexpr int FAST_RS_TABLE[] = {PA_FAST_RS_TABLE};
+constexpr int FAST_RS_BINARY[] = {PA_FAST_RS_BINARY};
 
 struct LaunchSpec {
     int loc, dir, gap, form, tr, R;
-    bool fastmax;   // v_max_f32 is exact (local maximize score, NaN-free table)
+    bool fastmax;   // the score kernel (max / min folds; R from the groups)
     int grid;       // workgroups of 256 threads (persistent)
     size_t lds_bytes;
     int pair;       // fast kernel: LDS table of row-symbol pairs (K1^2 * (K1-1) float2)
     int block;      // threads per workgroup
+    int var;        // VAR_*
 };
 // largest pair table the fast kernel stages (two workgroups per CU still fit)
 constexpr size_t PAIR_LDS_MAX = 80 * 1024;
@@ -292,7 +300,7 @@ struct WsbPlan {
 hipError_t launch_wsb_blocks(int loc, int dir, int form, const KArgs &args, const WsbPlan &plan, const float *ws,
                              const float *wt, int32_t *path, const int64_t *path_off, int32_t *path_len,
                              hipStream_t stream);
-bool supported_R(int form, int tr, bool fastmax, int R);
+bool supported_R(int form, int tr, int R);
 // The allocation-free entry point's device memory: a file-scope device array
 // of NOALLOC_SCRATCH_BYTES per GPU.  noalloc_scratch gives the current
 // device's copy (looked up once per device) and its CU count.

@@ -16,11 +16,11 @@
 // Every cell performs the reference's candidate fold in the reference's
 // order with strict-improvement updates (pyalign/algorithm/solver.h:1311-1427;
 // linear 2837-2854, Gotoh 2989-3035, DTW 3233-3250), so values are
-// bit-identical to the reference's float32 arithmetic.  The `FAST` variant
-// (local maximisation, score only, NaN-free table) uses v_max_f32: there
-// every value is >= +0 and no -0 can arise (the zero candidate is first and
-// a -0 never beats it, and +0 + -0 = +0), so max returns exactly the value
-// the strict select keeps.
+// bit-identical to the reference's float32 arithmetic.  Where no candidate can
+// be -0 or NaN, max / min folds return the same bits in fewer instructions
+// (the caller checks that; the score kernel's local maximum
+// over a NaN-free table needs less: every value is >= +0 and no -0 can arise,
+// the zero candidate being first, a -0 never beating it, and +0 + -0 = +0).
 #pragma once
 
 #include "pa_internal.h"
@@ -36,6 +36,11 @@ __device__ __forceinline__ bool better(float a, float b) {
 template <int DIR>
 __device__ __forceinline__ constexpr float worst() {
     return DIR == DIR_MAX ? -__builtin_inff() : __builtin_inff();
+}
+
+template <int DIR>
+__device__ __forceinline__ float opt(float a, float b) {
+    return DIR == DIR_MAX ? fmaxf(a, b) : fminf(a, b);
 }
 
 // lane k <- lane k-1 (wave_shr:1); lane 0 keeps its own value
@@ -88,7 +93,7 @@ __device__ __forceinline__ void band_wait(const KArgs &a, int idx, uint32_t need
 
 extern __shared__ float pa_dyn_lds[];  // the launch's dynamic LDS (table or staging windows)
 
-template <int LOC, int DIR, int GAP, int FORM, int TR, int R, bool FAST, int SD, bool BAND = false>
+template <int LOC, int DIR, int GAP, int FORM, int TR, int R, int SD, int VAR, bool BAND = false>
 __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, const float *__restrict__ tab,
                                             int lane) {
     constexpr float W = worst<DIR>();
@@ -347,7 +352,7 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
             constexpr bool KEEPV = KM == 1;  // cell values stored (a.dvals set)
             // no traceback stored (a checkpointed forward's group): the codes are not computed
             constexpr bool NOTB = KM == 2 || KM == 4;
-            // DTW over finite series: min / max folds, codes from equality tests
+            // min / max folds, codes from equality tests (DTW: finite series)
             constexpr bool MXF = KM >= 3;
             const int j = s - l;
             const int tsym = cur.sym;
@@ -398,7 +403,10 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
                     // search (the searches test rv), so its value is free except
                     // for the score-only local maximum, which folds every row:
                     // there it reads the worst similarity.
-                    constexpr bool PADW = LOC == LOC_LOCAL && TR == TR_SCORE;
+                    // (and the max-folding local search: the column's best row is
+                    // sought over every row, and a row that scores the worst
+                    // similarity never exceeds the last valid row above it)
+                    constexpr bool PADW = LOC == LOC_LOCAL && (TR == TR_SCORE || MXF);
                     float S;
                     if constexpr (TABLE) {
                         S = tab[rowsym[r] + tsym];
@@ -444,8 +452,10 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
                         const float dg = Dd + S;
                         const float up = Dup + go_s;
                         const float lf = Din[r] + go_t;
-                        if constexpr (FAST) {
-                            D = fmaxf(fmaxf(fmaxf(dg, 0.0f), up), lf);
+                        if constexpr (MXF) {
+                            D = opt<DIR>(opt<DIR>(LOC == LOC_LOCAL ? opt<DIR>(dg, 0.0f) : dg, up), lf);
+                            bits = dg == D ? 1u : (up == D ? 2u : 3u);
+                            if constexpr (LOC == LOC_LOCAL) bits = D == 0.0f ? 0u : bits;
                         } else {
                             int src;
                             if constexpr (LOC == LOC_LOCAL) {
@@ -468,10 +478,13 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
                         const float po = Dup + go_s, pe = Pup + ge_s;
                         const float qo = Din[r] + go_t, qe = Ql[r] + ge_t;
                         const float dg = Dd + S;
-                        if constexpr (FAST) {
-                            P = fmaxf(po, pe);
-                            Q = fmaxf(qo, qe);
-                            D = fmaxf(fmaxf(fmaxf(dg, 0.0f), P), Q);
+                        if constexpr (MXF) {
+                            P = opt<DIR>(po, pe);
+                            Q = opt<DIR>(qo, qe);
+                            D = opt<DIR>(opt<DIR>(LOC == LOC_LOCAL ? opt<DIR>(dg, 0.0f) : dg, P), Q);
+                            bits = dg == D ? 1u : (P == D ? 2u : 3u);
+                            if constexpr (LOC == LOC_LOCAL) bits = D == 0.0f ? 0u : bits;
+                            bits |= (better<DIR>(pe, po) ? 4u : 0u) | (better<DIR>(qe, qo) ? 8u : 0u);
                         } else {
                             const bool pext = better<DIR>(pe, po);
                             P = pext ? pe : po;
@@ -503,9 +516,8 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
                         if constexpr (TR == TR_SCORE) {
                             // pad rows never exceed the optimum: their S is the
                             // worst value and gap costs are non-negative
-                            if constexpr (FAST) best = fmaxf(best, D);
-                            else best = better<DIR>(D, best) ? D : best;
-                        } else {
+                            best = better<DIR>(D, best) ? D : best;
+                        } else if constexpr (!MXF) {
                             // Optima over i desc, j desc, first strict optimum
                             // wins (solver.h:2050-2056): largest i, then largest j
                             if (rv[r] && (better<DIR>(D, best) || (D == best && i >= bi))) {
@@ -558,6 +570,23 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
                     }
                 }
 
+                if constexpr (LOC == LOC_LOCAL && TR == TR_ONE && MXF) {
+                    // the column's best value; a lane looks for its row (the
+                    // lowest of equals) only where that may be a new best
+                    float m = Dout[0];
+#pragma unroll
+                    for (int r = 1; r < R; ++r) m = opt<DIR>(m, Dout[r]);
+                    if (!better<DIR>(best, m)) {
+                        int i = -1;
+#pragma unroll
+                        for (int r = 0; r < R; ++r) i = rv[r] && Dout[r] == m ? row0 + r : i;
+                        if (i >= 0 && (better<DIR>(m, best) || i >= bi)) {
+                            best = m;
+                            bi = i;
+                            bj = j;
+                        }
+                    }
+                }
                 // ---- seeds from the finished column (global / semiglobal) --
                 // (global: D(ls-1, lt-1) is read once the strip is done)
                 if constexpr (LOC == LOC_SEMI) {
@@ -568,7 +597,7 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
                         // last row, j ascending, strict (solver.h:2285-2287)
                         if (better<DIR>(v, rbest)) { rbest = v; rj = j; }
                     }
-                    if (j == lt - 1) {
+                    if (!STEADY && j == lt - 1) {  // (steady columns are never the last)
                         // last column, i ascending, strict (solver.h:2289-2291)
 #pragma unroll
                         for (int r = 0; r < R; ++r)
@@ -580,9 +609,12 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
         using std::integral_constant;
         // the step loop, built once per kind of group so that the usual loop
         // carries no per-cell test: 0 codes stored, 1 codes and cell values
-        // (a.dvals), 2 neither (the groups of a checkpointed forward keep
-        // strip rows only; their folds keep their order, their codes go);
-        // 3 and 4 as 0 and 2 for DTW over finite series, with min / max folds
+        // (a.dvals; kernels of their own, VAR_VALUES), 2 neither (the groups of
+        // a checkpointed forward keep strip rows only; their folds keep their
+        // order, their codes go); 3 and 4 as 0 and 2 with min / max folds (DTW
+        // over finite series; alignment over tables and binary symbols in
+        // kernels of their own, VAR_MAX: a kernel holds the registers of its
+        // largest loop, 256 and a wave per SIMD where these shared one)
         using Gen = integral_constant<bool, false>;
         auto sweep = [&](auto kv) {
             int s = 0;
@@ -626,13 +658,15 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
                 if (s < steps) step(Gen{}, integral_constant<int, 0>{}, kv, s, DlA, DlB, cA);
             }
         };
-        if constexpr (TR == TR_ONE) {
+        if constexpr (VAR == VAR_VALUES) {
+            sweep(integral_constant<int, 1>{});
+        } else if constexpr (VAR == VAR_MAX) {
+            sweep(integral_constant<int, 3>{});
+        } else if constexpr (TR == TR_ONE) {
             const bool notb = a.probs[g.first].tb_off == NO_TB_OFF;  // (one problem a group)
             bool mx = false;
             if constexpr (GAP == GAP_DTW && FORM == F_SERIES) mx = a.finite != nullptr && *a.finite != 0u;
-            if (a.dvals != nullptr) {
-                sweep(integral_constant<int, 1>{});
-            } else if (mx) {
+            if (mx) {
                 if constexpr (GAP == GAP_DTW && FORM == F_SERIES) {
                     if (notb) sweep(integral_constant<int, 4>{});
                     else sweep(integral_constant<int, 3>{});
@@ -642,9 +676,6 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
             } else {
                 sweep(integral_constant<int, 0>{});
             }
-        } else if constexpr (TR != TR_SCORE) {
-            if (a.dvals != nullptr) sweep(integral_constant<int, 1>{});
-            else sweep(integral_constant<int, 0>{});
         } else if constexpr (GAP == GAP_DTW && FORM == F_SERIES) {
             if (a.finite != nullptr && *a.finite != 0u) sweep(integral_constant<int, 3>{});  // (no codes to compute)
             else sweep(integral_constant<int, 0>{});
@@ -674,8 +705,7 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
         for (int m = 1; m < L; m <<= 1) {
             const float ob = __shfl_xor(best, m, WAVE);
             if constexpr (TR == TR_SCORE) {
-                if constexpr (FAST) best = fmaxf(best, ob);
-                else best = better<DIR>(ob, best) ? ob : best;
+                best = better<DIR>(ob, best) ? ob : best;
             } else {
                 const int oi = __shfl_xor(bi, m, WAVE);
                 const int oj = __shfl_xor(bj, m, WAVE);
@@ -739,37 +769,48 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
 }
 
 // ---------------------------------------------------------------------------
-// The score-only local maximisation path over a LDS table (the batched local
-// Gotoh / Smith-Waterman workload).  Same decomposition as solve_group with
-// the traceback and seed bookkeeping removed: every value is >= +0, so
-// v_max_f32 reproduces the strict select exactly (see the file comment),
-// the local borders are +0, and the optimum is a plain running maximum
-// (padded rows read the pad symbol, whose worst-valued entries keep them
-// below the optimum).  The column's symbol is loaded one step ahead.
+// The score kernel: score-only alignment over an LDS table or binary symbols
+// where max / min folds return the strict folds' bits (local maximisation
+// over a NaN-free table, see the file comment; elsewhere similarities finite
+// and no candidate -0, checked on the host).  Same decomposition as
+// solve_group with the traceback and seed positions removed; one kernel
+// serves every strip height from one queue.
 //
-// Gotoh here carries P' = max(P, 0) and Q' = max(Q, 0) instead of P and Q:
+// Local Gotoh carries P' = max(P, 0) and Q' = max(Q, 0) instead of P and Q:
 // with a non-positive extension term e, max(0, max(P, 0) + e) =
 // max(0, P + e), so P'(i) = max(0, D(i-1) + o, P'(i-1) + e) = max(0, P(i))
 // by induction (the same float additions whenever P >= 0, both sides
 // clamped to 0 otherwise), and D = max(0, diag, P, Q) = max3(diag, P', Q'):
-// one v_max3_f32 per layer instead of a separate zero clamp.
+// one v_max3_f32 per layer instead of a separate zero clamp (minimising: the
+// mirror image).
 //
 // The left column D(i, j-1) lives in two register banks used alternately
 // by consecutive steps (steps go in pairs): row r+1 still needs the old
 // D(i, j-1) of row r as its diagonal after row r's new value exists, so a
 // single bank would cost a register copy per cell.  Both banks start at the
 // border value and a lane leaves them untouched while it waits for its
-// first column, so whichever bank a step reads holds the border.
+// first column, so whichever bank a step reads holds the border; nor does it
+// touch them after its last column, so that the strip's last column is read
+// from them once the strip is done (global corner, semiglobal last column).
 //
-// PAIR: the LDS holds the table for row-symbol pairs, entry ((x1 * K1 + x2)
-// * Kc + y) = (S(x1, y), S(x2, y)) with Kc = K1 - 1 real column symbols, so
-// rows 2q and 2q+1 of a lane get their similarities from one ds_read_b64 at
+// SRC_PAIR: the LDS holds the table for row-symbol pairs, entry ((x1 * K1 +
+// x2) * Kc + y) = (S(x1, y), S(x2, y)) with Kc = K1 - 1 real column symbols,
+// so rows 2q and 2q+1 of a lane get their similarities from one ds_read_b64 at
 // one address add (K1^2 * Kc * 8 bytes: 70,560 for 20 symbols and the pad).
+//
+// Bound by VALU issue.  Kernel times on one MI355X: 65,536 local Gotoh pairs of
+// 50 to 2,000 over a table 3.7 ms; 16,384 global affine pairs of 50 to 1,000
+// 0.5 ms (the general kernel's strict folds with long mode 8.6 ms); 16,384
+// semiglobal affine pairs of 125 x 300 binary symbols 0.29 ms (0.51 ms).
 // ---------------------------------------------------------------------------
-template <int GAP, bool PAIR, int R>
+enum { SRC_TABLE = 0, SRC_PAIR = 1, SRC_BINARY = 2 };
+
+template <int LOC, int DIR, int GAP, int SRC, int R>
 __device__ __forceinline__ void solve_group_fast(const KArgs &a, const Group &g, const float *__restrict__ tab,
                                                  int lane) {
-    constexpr float NEG = -__builtin_inff();
+    constexpr float W = worst<DIR>();
+    constexpr bool LOCAL = LOC == LOC_LOCAL, GLOBAL = LOC == LOC_GLOBAL, SEMI = LOC == LOC_SEMI;
+    constexpr bool PAIR = SRC == SRC_PAIR, BINARY = SRC == SRC_BINARY;
     const int L = g.L;
     const int seg = lane >> g.lgL;
     const int l = lane & (L - 1);
@@ -791,9 +832,18 @@ __device__ __forceinline__ void solve_group_fast(const KArgs &a, const Group &g,
     const int K1 = a.K1;
     const int PAD = K1 - 1;
     const float go_s = a.go_s, ge_s = a.ge_s, go_t = a.go_t, ge_t = a.ge_t;
-    const uint8_t *__restrict__ cs = (const uint8_t *)a.codes_s;
-    const uint8_t *__restrict__ ct = (const uint8_t *)a.codes_t;
-    float best = NEG;
+    const float eq = a.eq, ne = a.ne;
+    using Code = std::conditional_t<BINARY, uint32_t, uint8_t>;
+    const Code *__restrict__ cs = (const Code *)a.codes_s;
+    const Code *__restrict__ ct = (const Code *)a.codes_t;
+    float best = W;  // local: over all cells; semiglobal: over the last column
+    [[maybe_unused]] float rbest = W;   // semiglobal: over the last row
+    [[maybe_unused]] float corner = W;  // global
+    // the last row's strip, lane and row in the lane
+    const int last = ls - 1;
+    [[maybe_unused]] const int st_last = last >= 0 ? last / rps : -1;
+    [[maybe_unused]] const int l_last = last >= 0 ? (last % rps) / R : -1;
+    [[maybe_unused]] const int r_last = last >= 0 ? last % R : -1;
     // steady steps: the members' shortest length and fewest strips, and safe
     // symbol addresses (the first member's) for lanes without a member
     int min_lt = has ? lt : 0x7fffffff, min_nst = has ? nst : 0x7fffffff;
@@ -803,63 +853,91 @@ __device__ __forceinline__ void solve_group_fast(const KArgs &a, const Group &g,
     }
     min_lt = __builtin_amdgcn_readfirstlane(min_lt);  // the same in every lane
     min_nst = __builtin_amdgcn_readfirstlane(min_nst);
-    // index of the symbol of column s - l + 1 is t_ix + s
-    const int64_t t_ix = (has ? off_t : a.probs[g.first].off_t) + 1 - l;
+    // loads two steps ahead; tall strips, whose steps are long and whose
+    // registers are full, one (65,536 local pairs, mostly tall: no difference)
+    constexpr int AHEAD = R <= 16 ? 2 : 1;
+    // index of the symbol of column s - l + AHEAD is t_ix + s
+    const int64_t t_ix = (has ? off_t : a.probs[g.first].off_t) + AHEAD - l;
 
     for (int st = 0; st < g.max_nst; ++st) {
         const bool act = st < nst;
-        const bool rd_top = has && l == 0 && st > 0;         // lane 0 reads the strip above's row
+        // lane 0 reads the row above: the strip above's, or the global border
+        const bool rd_top = has && l == 0 && (GLOBAL || st > 0);
         const bool wr_bot = l == L - 1 && st + 1 < nst;      // the last lane writes it for the next
         const int row0 = st * rps + l * R;
         int rowsym[R];
         [[maybe_unused]] int rowpair[R / 2 > 0 ? R / 2 : 1];
+        // local binary: a padded row never scores eq (its value stays below the optimum)
+        [[maybe_unused]] float eqr[BINARY && LOCAL ? R : 1];
         float DlA[R], DlB[R], Ql[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int i = row0 + r;
-            rowsym[r] = ((act && i < ls) ? int(cs[off_s + i]) : PAD) * K1;
-            DlA[r] = 0.0f;  // local border D(i, -1) = +0 (solver.h:2021-2029)
-            DlB[r] = 0.0f;
-            Ql[r] = NEG;    // Q(i, -1)
+            const bool rv = act && i < ls;
+            if constexpr (BINARY) {
+                rowsym[r] = rv ? int(cs[off_s + i]) : 0;
+                if constexpr (LOCAL) eqr[r] = rv ? eq : ne;
+            } else {
+                rowsym[r] = (rv ? int(cs[off_s + i]) : PAD) * K1;
+            }
+            // D(i, -1): local and semiglobal +0 (solver.h:2021-2029, 2253-2261)
+            DlA[r] = GLOBAL ? (rv ? a.border_s[i + 1] : W) : 0.0f;
+            DlB[r] = DlA[r];
+            Ql[r] = W;    // Q(i, -1)
         }
         if constexpr (PAIR) {
             // byte offset of the (row 2q, row 2q+1) symbol pair's block
 #pragma unroll
             for (int q = 0; q < R / 2; ++q) rowpair[q] = (rowsym[2 * q] + rowsym[2 * q + 1] / K1) * (K1 - 1) * 8;
         }
-        float botD = 0.0f, botP = NEG;
-        float prevD = 0.0f;  // D(row0-1, -1) = +0
-        // global memory is touched only at the top of a step, one step
-        // ahead: the column's symbol and (lane 0) the row above the strip are
-        // loaded for the next step, and the last lane's bottom row of the
-        // previous step is stored, so every load and store has a whole step
-        // of cells to complete before anything waits on it
-        int tnext = 0;
-        if (act && l == 0 && lt > 0) tnext = int(ct[off_t]);
-        // lane 0's row above, loaded a step ahead into alternating registers
-        // (a step reads one and loads the other: no copies between steps)
-        float2 nxA = make_float2(0.0f, NEG), nxB = nxA;  // D(-1, j) = +0, P(-1, j) = worst on the first strip
-        if (l == 0 && st > 0 && act && lt > 0) nxA = a.rowbuf[rb_off];
+        float botD = DlA[R - 1], botP = W;
+        float prevD = 0.0f;  // D(row0-1, -1)
+        if constexpr (GLOBAL)
+            prevD = l == 0 && act ? (row0 == 0 ? a.border_t[0] : a.border_s[row0]) : W;
+        // global memory is touched only at the top of a step: the column's
+        // symbol and (lane 0) the row above the strip are loaded AHEAD steps
+        // before their use into one of two slots used alternately, and the
+        // last lane's bottom row of the previous step is stored, so every load
+        // and store has a whole step of cells or more to complete before
+        // anything waits on it
+        int tA = 0, tB = 0;
+        // D(-1, j) = +0 or the global border, P(-1, j) = worst on the first strip
+        float2 nxA = make_float2(0.0f, W), nxB = nxA;
+        auto above = [&](int64_t j, float2 &nx) {  // column j
+            if (GLOBAL && st == 0) nx.x = a.border_t[j + 1];
+            else nx = a.rowbuf[rb_off + j];
+        };
+        if (act && l == 0 && lt > 0) tA = int(ct[off_t]);
+        if (rd_top && act && lt > 0) above(0, nxA);
+        if constexpr (AHEAD == 2) {
+            if (act && l < 2 && lt > 1 - l) tB = int(ct[off_t + 1 - l]);
+            if (rd_top && act && lt > 1) above(1, nxB);
+        }
         bool pend = false;  // a bottom row value waiting to be stored
         float2 pendv = make_float2(0.0f, 0.0f);
         int pendj = 0;
+        [[maybe_unused]] const bool last_row = SEMI && act && st == st_last && l == l_last;
 
         // one step: column j = s - l of this lane's R rows, left column read
-        // from Din, this column written to Dout.  A steady step (every lane of
-        // every member inside its problem's strip and columns, the next column
-        // too) drops the range tests; lanes without a member read the first
-        // member's symbols and discard what they compute.
-        auto step = [&](auto steady, int s, float (&Din)[R], float (&Dout)[R], const float2 &nxin, float2 &nxout) {
+        // from Din, this column written to Dout, the column's inputs in slot
+        // (tc, nxc), the next step's in (tn, nxn).  A steady step (every lane
+        // of every member inside its problem's strip and columns, the column
+        // it loads too) drops the range tests; lanes without a member read the
+        // first member's symbols and discard what they compute.
+        auto step = [&](auto steady, int s, float (&Din)[R], float (&Dout)[R], int &tc, float2 &nxc, int &tn,
+                        float2 &nxn) {
             constexpr bool STEADY = decltype(steady)::value;
             const int j = s - l;
-            const int tsym = tnext;
-            const float rD = nxin.x, rP = nxin.y;
+            const int tsym = tc;
+            const float rD = nxc.x, rP = nxc.y;
+            int &tl = AHEAD == 2 ? tc : tn;  // the slot of step s + AHEAD
+            float2 &nxl = AHEAD == 2 ? nxc : nxn;
             if constexpr (STEADY) {
-                tnext = int(ct[t_ix + s]);
-                if (rd_top) nxout = a.rowbuf[rb_off + 1 + s];  // lane 0: column s + 1
+                tl = int(ct[t_ix + s]);
+                if (rd_top) above(AHEAD + s, nxl);  // lane 0: column s + AHEAD
             } else {
-                if (act && j + 1 >= 0 && j + 1 < lt) tnext = int(ct[off_t + j + 1]);
-                if (l == 0 && st > 0 && act && j + 1 < lt) nxout = a.rowbuf[rb_off + j + 1];
+                if (act && j + AHEAD >= 0 && j + AHEAD < lt) tl = int(ct[off_t + j + AHEAD]);
+                if (rd_top && act && j + AHEAD < lt) above(j + AHEAD, nxl);
             }
             if (pend) {  // after the loads: the next wait on them need not wait for it
                 if constexpr (STEADY) a.rowbuf[rb_off - 1 - l + s] = pendv;  // column s - 1 - l
@@ -891,25 +969,41 @@ __device__ __forceinline__ void solve_group_fast(const KArgs &a, const Group &g,
                 for (int r = 0; r < R; ++r) {
                     float S;
                     if constexpr (PAIR) S = Sv[r];
+                    else if constexpr (BINARY) S = rowsym[r] == tsym ? (LOCAL ? eqr[r] : eq) : ne;
                     else S = tab[rowsym[r] + tsym];
                     const float dg = Dd + S;
                     float D;
                     if constexpr (GAP == GAP_AFF) {
-                        const float Pc = fmaxf(fmaxf(Gup, Pup + ge_s), 0.0f);
-                        const float Qc = fmaxf(fmaxf(Din[r] + go_t, Ql[r] + ge_t), 0.0f);
-                        D = fmaxf(fmaxf(dg, Pc), Qc);
+                        float Pc = opt<DIR>(Gup, Pup + ge_s);
+                        float Qc = opt<DIR>(Din[r] + go_t, Ql[r] + ge_t);
+                        if constexpr (LOCAL) {
+                            Pc = opt<DIR>(Pc, 0.0f);
+                            Qc = opt<DIR>(Qc, 0.0f);
+                        }
+                        D = opt<DIR>(opt<DIR>(dg, Pc), Qc);
                         Ql[r] = Qc;
                         Pup = Pc;
                     } else {
-                        D = fmaxf(fmaxf(fmaxf(dg, 0.0f), Gup), Din[r] + go_t);
+                        if constexpr (LOCAL) D = opt<DIR>(opt<DIR>(opt<DIR>(dg, 0.0f), Gup), Din[r] + go_t);
+                        else D = opt<DIR>(opt<DIR>(dg, Gup), Din[r] + go_t);
                     }
-                    best = fmaxf(best, D);
+                    if constexpr (LOCAL) best = opt<DIR>(best, D);
                     Dd = Din[r];
                     Dout[r] = D;
                     Gup = D + go_s;
                 }
                 botD = Dout[R - 1];
                 botP = Pup;
+                if constexpr (SEMI) {
+                    if (last_row) {
+                        float v = Dout[0];
+                        int rl = r_last;  // (its tests stay here: kept as R lane masks they spill)
+                        asm("" : "+v"(rl));
+#pragma unroll
+                        for (int r = 1; r < R; ++r) v = r == rl ? Dout[r] : v;
+                        rbest = opt<DIR>(rbest, v);
+                    }
+                }
                 if constexpr (STEADY) {  // pendv is read only where pend is set
                     pend = wr_bot;
                     pendv = make_float2(botD, botP);
@@ -923,40 +1017,78 @@ __device__ __forceinline__ void solve_group_fast(const KArgs &a, const Group &g,
         using General = std::integral_constant<bool, false>;
         using Steady = std::integral_constant<bool, true>;
         // steps [sa, sb) are steady: s >= L - 1 puts every lane at a column
-        // >= 0, s + 1 < the members' shortest length keeps every lane's next
-        // column inside its member (only when every member still has this
+        // >= 0, s + AHEAD < the members' shortest length keeps every column a
+        // lane loads inside its member (only when every member still has this
         // strip); both ends are even so the register banks keep their order
         const int sa = L & ~1;
-        const int sb = st < min_nst ? ((min_lt - 1) & ~1) : 0;
+        const int sb = st < min_nst ? ((min_lt - AHEAD) & ~1) : 0;
         int s = 0;
         if (sa < sb) {
             for (; s < sa; s += 2) {
-                step(General{}, s, DlA, DlB, nxA, nxB);
-                step(General{}, s + 1, DlB, DlA, nxB, nxA);
+                step(General{}, s, DlA, DlB, tA, nxA, tB, nxB);
+                step(General{}, s + 1, DlB, DlA, tB, nxB, tA, nxA);
             }
             for (int k = (sb - sa) >> 1; k > 0; --k, s += 2) {  // a uniform trip count
-                step(Steady{}, s, DlA, DlB, nxA, nxB);
-                step(Steady{}, s + 1, DlB, DlA, nxB, nxA);
+                step(Steady{}, s, DlA, DlB, tA, nxA, tB, nxB);
+                step(Steady{}, s + 1, DlB, DlA, tB, nxB, tA, nxA);
             }
             pendj = s - 1 - l;  // the column of a store still pending
         }
         for (; s + 1 < steps; s += 2) {
-            step(General{}, s, DlA, DlB, nxA, nxB);
-            step(General{}, s + 1, DlB, DlA, nxB, nxA);
+            step(General{}, s, DlA, DlB, tA, nxA, tB, nxB);
+            step(General{}, s + 1, DlB, DlA, tB, nxB, tA, nxA);
         }
-        if (s < steps) step(General{}, s, DlA, DlB, nxA, nxB);
+        if (s < steps) step(General{}, s, DlA, DlB, tA, nxA, tB, nxB);
         if (pend) a.rowbuf[rb_off + pendj] = pendv;
+        // the last column: step lt-1+l wrote DlB when even and DlA when odd
+        if constexpr (!LOCAL) {
+            const bool odd = ((lt - 1 + l) & 1) != 0;
+            if (act && (SEMI || (st == st_last && l == l_last))) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const float v = odd ? DlA[r] : DlB[r];
+                    if (SEMI) best = row0 + r < ls ? opt<DIR>(best, v) : best;
+                    else corner = r == r_last ? v : corner;
+                }
+            }
+        }
         __threadfence_block();
     }
-    for (int m = 1; m < L; m <<= 1) best = fmaxf(best, __shfl_xor(best, m, WAVE));
-    if (has && l == 0) a.scores[out] = (ls == 0 || lt == 0) ? NEG : best;
+    float score;
+    if constexpr (GLOBAL) {
+        score = __shfl(corner, (seg << g.lgL) + max(l_last, 0), WAVE);
+    } else {
+        for (int m = 1; m < L; m <<= 1) best = opt<DIR>(best, __shfl_xor(best, m, WAVE));
+        score = best;
+        if constexpr (SEMI) score = opt<DIR>(best, __shfl(rbest, (seg << g.lgL) + max(l_last, 0), WAVE));
+    }
+    if (has && l == 0) {
+        if (LOCAL) a.scores[out] = (ls == 0 || lt == 0) ? W : score;
+        else if (ls == 0 || lt == 0) write_empty<LOC, DIR>(a, a.probs[g.first + seg]);
+        else a.scores[out] = score;
+    }
 }
 
-template <int GAP, bool PAIR, int... RS>
+// A wavefront's groups: the first by its place in the grid (the longest groups,
+// queued first, one to a workgroup), the others from the ticket counter.  A
+// counter that every wavefront starts with is one address that thousands of
+// atomics queue for.
+// Band-mode strips wait for one another and are taken in order throughout.
+__device__ __forceinline__ uint32_t next_ticket(const KArgs &a, int lane) {
+    uint32_t t = 0;
+    if (lane == 0) t = atomicAdd(a.queue, 1u) + (a.progress ? 0u : gridDim.x * (blockDim.x / WAVE));
+    return uint32_t(__builtin_amdgcn_readlane(int(t), 0));  // uniform: the group's fields load as scalars
+}
+__device__ __forceinline__ uint32_t first_ticket(const KArgs &a) {
+    if (a.progress) return next_ticket(a, int(threadIdx.x) & (WAVE - 1));
+    return uint32_t(__builtin_amdgcn_readfirstlane(int((threadIdx.x / WAVE) * gridDim.x + blockIdx.x)));
+}
+
+template <int LOC, int DIR, int GAP, int SRC, int... RS>
 __global__ __launch_bounds__(FAST_BLOCK) void pa_fast_kernel(KArgs a) {
     extern __shared__ float lds_table[];
     const int K1 = a.K1;
-    if constexpr (PAIR) {
+    if constexpr (SRC == SRC_PAIR) {
         const int Kc = K1 - 1;
         const int n = K1 * K1 * Kc;
         float2 *pt = reinterpret_cast<float2 *>(lds_table);
@@ -964,26 +1096,22 @@ __global__ __launch_bounds__(FAST_BLOCK) void pa_fast_kernel(KArgs a) {
             const int y = k % Kc, p = k / Kc;
             pt[k] = make_float2(a.table[(p / K1) * K1 + y], a.table[(p % K1) * K1 + y]);
         }
-    } else {
+    } else if constexpr (SRC == SRC_TABLE) {
         const int n = K1 * K1;
         for (int k = threadIdx.x; k < n; k += blockDim.x) lds_table[k] = a.table[k];
     }
     __syncthreads();
     const int lane = threadIdx.x & (WAVE - 1);
-    while (true) {
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(a.queue, 1u);
-        t = uint32_t(__builtin_amdgcn_readlane(int(t), 0));  // uniform: the group's fields load as scalars
-        if (t >= uint32_t(a.n_groups)) break;
+    for (uint32_t t = first_ticket(a); t < uint32_t(a.n_groups); t = next_ticket(a, lane)) {
         const Group &g = a.groups[t];
         const int R = g.R;
-        (void)((R == RS ? (solve_group_fast<GAP, PAIR, RS>(a, g, lds_table, lane), true) : false) || ...);
+        (void)((R == RS ? (solve_group_fast<LOC, DIR, GAP, SRC, RS>(a, g, lds_table, lane), true) : false) || ...);
     }
 }
 
-template <int GAP, bool PAIR>
+template <int LOC, int DIR, int GAP, int SRC, int... RS>
 static hipError_t go_fast_t(const LaunchSpec &s, const KArgs &a, hipStream_t st, int *occ_out) {
-    const void *fn = reinterpret_cast<const void *>(&pa_fast_kernel<GAP, PAIR, PA_FAST_RS_LIST>);
+    const void *fn = reinterpret_cast<const void *>(&pa_fast_kernel<LOC, DIR, GAP, SRC, RS...>);
     if (occ_out) {
         int blocks = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, fn, FAST_BLOCK, s.lds_bytes) != hipSuccess)
@@ -992,16 +1120,23 @@ static hipError_t go_fast_t(const LaunchSpec &s, const KArgs &a, hipStream_t st,
         return hipSuccess;
     }
     const int block = s.block > 0 && s.block <= FAST_BLOCK && s.block % WAVE == 0 ? s.block : 256;
-    hipLaunchKernelGGL((pa_fast_kernel<GAP, PAIR, PA_FAST_RS_LIST>), dim3(s.grid), dim3(block), s.lds_bytes, st, a);
+    hipLaunchKernelGGL((pa_fast_kernel<LOC, DIR, GAP, SRC, RS...>), dim3(s.grid), dim3(block), s.lds_bytes, st, a);
     return hipGetLastError();
 }
 
-template <int GAP>
+template <int LOC, int DIR, int GAP>
 static hipError_t go_fast(const LaunchSpec &s, const KArgs &a, hipStream_t st, int *occ_out) {
-    return s.pair ? go_fast_t<GAP, true>(s, a, st, occ_out) : go_fast_t<GAP, false>(s, a, st, occ_out);
+    if (s.form == F_BINARY) return go_fast_t<LOC, DIR, GAP, SRC_BINARY, PA_FAST_RS_BINARY>(s, a, st, occ_out);
+    if constexpr (LOC == LOC_LOCAL && DIR == DIR_MAX) {
+        return s.pair ? go_fast_t<LOC, DIR, GAP, SRC_PAIR, PA_FAST_RS_LIST>(s, a, st, occ_out)
+                      : go_fast_t<LOC, DIR, GAP, SRC_TABLE, PA_FAST_RS_LIST>(s, a, st, occ_out);
+    } else {
+        return s.pair ? go_fast_t<LOC, DIR, GAP, SRC_PAIR, PA_FAST_RS_TABLE>(s, a, st, occ_out)
+                      : go_fast_t<LOC, DIR, GAP, SRC_TABLE, PA_FAST_RS_TABLE>(s, a, st, occ_out);
+    }
 }
 
-template <int LOC, int DIR, int GAP, int FORM, int TR, int R, bool FAST, int SD>
+template <int LOC, int DIR, int GAP, int FORM, int TR, int R, int SD, int VAR>
 __global__ __launch_bounds__(256) void pa_solve_kernel(KArgs a) {
     extern __shared__ float lds_table[];
     if constexpr (FORM == F_TABLE) {
@@ -1014,34 +1149,30 @@ __global__ __launch_bounds__(256) void pa_solve_kernel(KArgs a) {
     const int lane = threadIdx.x & (WAVE - 1);
     // Persistent wavefronts drain the cost-sorted group queue; every wave
     // leaves once its ticket passes the group count.
-    while (true) {
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(a.queue, 1u);
-        t = uint32_t(__builtin_amdgcn_readlane(int(t), 0));  // uniform: the group's fields load as scalars
-        if (t >= uint32_t(a.n_groups)) break;
+    for (uint32_t t = first_ticket(a); t < uint32_t(a.n_groups); t = next_ticket(a, lane)) {
         const Group &g = a.groups[t];
-        if constexpr (!FAST && TR != TR_ALL) {
+        if constexpr (TR != TR_ALL) {
             if (g.strip >= 0) {
-                solve_group<LOC, DIR, GAP, FORM, TR, R, FAST, SD, true>(a, g, tab, lane);
+                solve_group<LOC, DIR, GAP, FORM, TR, R, SD, VAR, true>(a, g, tab, lane);
                 continue;
             }
         }
-        solve_group<LOC, DIR, GAP, FORM, TR, R, FAST, SD>(a, g, tab, lane);
+        solve_group<LOC, DIR, GAP, FORM, TR, R, SD, VAR>(a, g, tab, lane);
     }
 }
 
-template <int LOC, int DIR, int GAP, int FORM, int TR, int R, bool FAST, int SD>
+template <int LOC, int DIR, int GAP, int FORM, int TR, int R, int SD, int VAR>
 static hipError_t go(const LaunchSpec &s, const KArgs &a, hipStream_t st) {
-    hipLaunchKernelGGL((pa_solve_kernel<LOC, DIR, GAP, FORM, TR, R, FAST, SD>), dim3(s.grid), dim3(256),
+    hipLaunchKernelGGL((pa_solve_kernel<LOC, DIR, GAP, FORM, TR, R, SD, VAR>), dim3(s.grid), dim3(256),
                        s.lds_bytes, st, a);
     return hipGetLastError();
 }
 
-template <int LOC, int DIR, int GAP, int FORM, int TR, int R, bool FAST, int SD>
+template <int LOC, int DIR, int GAP, int FORM, int TR, int R, int SD, int VAR>
 static int occ(const LaunchSpec &s) {
     int blocks = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &blocks, reinterpret_cast<const void *>(&pa_solve_kernel<LOC, DIR, GAP, FORM, TR, R, FAST, SD>), 256,
+            &blocks, reinterpret_cast<const void *>(&pa_solve_kernel<LOC, DIR, GAP, FORM, TR, R, SD, VAR>), 256,
             s.lds_bytes) != hipSuccess)
         return 4;
     return blocks * 4;
@@ -1051,101 +1182,86 @@ static int occ(const LaunchSpec &s) {
 // general strip height R = 8; the hot score-only table path gets more.
 template <int LOC, int DIR, int GAP, bool OCC>
 static hipError_t dispatch_lg(const LaunchSpec &s, const KArgs &a, hipStream_t st, int *occ_out) {
-#define PA_GO(FORM, TR, R, FAST, SD)                                                        \
-    do {                                                                                    \
-        if (OCC) {                                                                          \
-            *occ_out = occ<LOC, DIR, GAP, FORM, TR, R, FAST, SD>(s);                        \
-            return hipSuccess;                                                              \
-        }                                                                                   \
-        return go<LOC, DIR, GAP, FORM, TR, R, FAST, SD>(s, a, st);                          \
+#define PA_GO_VAR(FORM, TR, R, SD, VAR)                             \
+    do {                                                            \
+        if (OCC) {                                                  \
+            *occ_out = occ<LOC, DIR, GAP, FORM, TR, R, SD, VAR>(s); \
+            return hipSuccess;                                      \
+        }                                                           \
+        return go<LOC, DIR, GAP, FORM, TR, R, SD, VAR>(s, a, st);   \
+    } while (0)
+#define PA_GO(FORM, TR, R, SD)                                                                   \
+    do {                                                                                         \
+        if constexpr (TR != TR_SCORE)                                                            \
+            if (s.var == VAR_VALUES) PA_GO_VAR(FORM, TR, R, SD, VAR_VALUES);                     \
+        if constexpr (TR == TR_ONE && GAP != GAP_DTW && (FORM == F_TABLE || FORM == F_BINARY))   \
+            if (s.var == VAR_MAX) PA_GO_VAR(FORM, TR, R, SD, VAR_MAX);                           \
+        PA_GO_VAR(FORM, TR, R, SD, VAR_PLAIN);                                                   \
     } while (0)
     if constexpr (GAP == GAP_DTW) {
         if (s.tr == TR_ALL) return hipErrorInvalidValue;
         if (s.R != 8) return hipErrorInvalidValue;
         if (s.form == F_DENSE) {
-            if (s.tr == TR_SCORE) PA_GO(F_DENSE, TR_SCORE, 8, false, 0);
-            PA_GO(F_DENSE, TR_ONE, 8, false, 0);
+            if (s.tr == TR_SCORE) PA_GO(F_DENSE, TR_SCORE, 8, 0);
+            PA_GO(F_DENSE, TR_ONE, 8, 0);
         }
         if (s.form == F_DROWS) {
-            if (s.tr == TR_SCORE) PA_GO(F_DROWS, TR_SCORE, 8, false, 0);
-            PA_GO(F_DROWS, TR_ONE, 8, false, 0);
+            if (s.tr == TR_SCORE) PA_GO(F_DROWS, TR_SCORE, 8, 0);
+            PA_GO(F_DROWS, TR_ONE, 8, 0);
         }
         if (s.form == F_SERIES) {
             switch (a.dim) {
-                case 1: if (s.tr == TR_SCORE) PA_GO(F_SERIES, TR_SCORE, 8, false, 1); PA_GO(F_SERIES, TR_ONE, 8, false, 1);
-                case 2: if (s.tr == TR_SCORE) PA_GO(F_SERIES, TR_SCORE, 8, false, 2); PA_GO(F_SERIES, TR_ONE, 8, false, 2);
-                case 3: if (s.tr == TR_SCORE) PA_GO(F_SERIES, TR_SCORE, 8, false, 3); PA_GO(F_SERIES, TR_ONE, 8, false, 3);
-                case 4: if (s.tr == TR_SCORE) PA_GO(F_SERIES, TR_SCORE, 8, false, 4); PA_GO(F_SERIES, TR_ONE, 8, false, 4);
+                case 1: if (s.tr == TR_SCORE) PA_GO(F_SERIES, TR_SCORE, 8, 1); PA_GO(F_SERIES, TR_ONE, 8, 1);
+                case 2: if (s.tr == TR_SCORE) PA_GO(F_SERIES, TR_SCORE, 8, 2); PA_GO(F_SERIES, TR_ONE, 8, 2);
+                case 3: if (s.tr == TR_SCORE) PA_GO(F_SERIES, TR_SCORE, 8, 3); PA_GO(F_SERIES, TR_ONE, 8, 3);
+                case 4: if (s.tr == TR_SCORE) PA_GO(F_SERIES, TR_SCORE, 8, 4); PA_GO(F_SERIES, TR_ONE, 8, 4);
                 default: return hipErrorInvalidValue;
             }
         }
         return hipErrorInvalidValue;
     } else {
+        if (s.fastmax) return go_fast<LOC, DIR, GAP>(s, a, st, occ_out);
         if (s.form == F_TABLE && s.tr == TR_SCORE) {
-            if (s.fastmax) {
-                if constexpr (LOC == LOC_LOCAL && DIR == DIR_MAX) {
-                    if (s.R == 0) return go_fast<GAP>(s, a, st, occ_out);
-                    switch (s.R) {
-                        case 1: PA_GO(F_TABLE, TR_SCORE, 1, true, 0);
-                        case 2: PA_GO(F_TABLE, TR_SCORE, 2, true, 0);
-                        case 3: PA_GO(F_TABLE, TR_SCORE, 3, true, 0);
-                        case 4: PA_GO(F_TABLE, TR_SCORE, 4, true, 0);
-                        case 5: PA_GO(F_TABLE, TR_SCORE, 5, true, 0);
-                        case 6: PA_GO(F_TABLE, TR_SCORE, 6, true, 0);
-                        case 7: PA_GO(F_TABLE, TR_SCORE, 7, true, 0);
-                        case 8: PA_GO(F_TABLE, TR_SCORE, 8, true, 0);
-                        case 10: PA_GO(F_TABLE, TR_SCORE, 10, true, 0);
-                        case 12: PA_GO(F_TABLE, TR_SCORE, 12, true, 0);
-                        case 14: PA_GO(F_TABLE, TR_SCORE, 14, true, 0);
-                        case 16: PA_GO(F_TABLE, TR_SCORE, 16, true, 0);
-                        case 20: PA_GO(F_TABLE, TR_SCORE, 20, true, 0);
-                        case 24: PA_GO(F_TABLE, TR_SCORE, 24, true, 0);
-                        case 28: PA_GO(F_TABLE, TR_SCORE, 28, true, 0);
-                        case 32: PA_GO(F_TABLE, TR_SCORE, 32, true, 0);
-                        default: return hipErrorInvalidValue;
-                    }
-                }
-                return hipErrorInvalidValue;
-            }
             switch (s.R) {
-                case 4: PA_GO(F_TABLE, TR_SCORE, 4, false, 0);
-                case 8: PA_GO(F_TABLE, TR_SCORE, 8, false, 0);
-                case 16: PA_GO(F_TABLE, TR_SCORE, 16, false, 0);
-                case 32: PA_GO(F_TABLE, TR_SCORE, 32, false, 0);
+                case 4: PA_GO(F_TABLE, TR_SCORE, 4, 0);
+                case 8: PA_GO(F_TABLE, TR_SCORE, 8, 0);
+                case 16: PA_GO(F_TABLE, TR_SCORE, 16, 0);
+                case 32: PA_GO(F_TABLE, TR_SCORE, 32, 0);
                 default: return hipErrorInvalidValue;
             }
         }
         if (s.R == 4) {  // band-mode strips of a long problem (more, shorter strips)
-            if (s.form == F_TABLE && s.tr == TR_ONE) PA_GO(F_TABLE, TR_ONE, 4, false, 0);
-            if (s.form == F_BINARY && s.tr == TR_SCORE) PA_GO(F_BINARY, TR_SCORE, 4, false, 0);
-            if (s.form == F_BINARY && s.tr == TR_ONE) PA_GO(F_BINARY, TR_ONE, 4, false, 0);
+            if (s.form == F_TABLE && s.tr == TR_ONE) PA_GO(F_TABLE, TR_ONE, 4, 0);
+            if (s.form == F_BINARY && s.tr == TR_SCORE) PA_GO(F_BINARY, TR_SCORE, 4, 0);
+            if (s.form == F_BINARY && s.tr == TR_ONE) PA_GO(F_BINARY, TR_ONE, 4, 0);
             return hipErrorInvalidValue;
         }
         if (s.R != 8) return hipErrorInvalidValue;
         switch (s.form) {
             case F_TABLE:
-                if (s.tr == TR_ONE) PA_GO(F_TABLE, TR_ONE, 8, false, 0);
-                PA_GO(F_TABLE, TR_ALL, 8, false, 0);
+                if (s.tr == TR_ONE) PA_GO(F_TABLE, TR_ONE, 8, 0);
+                PA_GO(F_TABLE, TR_ALL, 8, 0);
             case F_TABLE_G:
-                if (s.tr == TR_SCORE) PA_GO(F_TABLE_G, TR_SCORE, 8, false, 0);
-                if (s.tr == TR_ONE) PA_GO(F_TABLE_G, TR_ONE, 8, false, 0);
-                PA_GO(F_TABLE_G, TR_ALL, 8, false, 0);
+                if (s.tr == TR_SCORE) PA_GO(F_TABLE_G, TR_SCORE, 8, 0);
+                if (s.tr == TR_ONE) PA_GO(F_TABLE_G, TR_ONE, 8, 0);
+                PA_GO(F_TABLE_G, TR_ALL, 8, 0);
             case F_BINARY:
-                if (s.tr == TR_SCORE) PA_GO(F_BINARY, TR_SCORE, 8, false, 0);
-                if (s.tr == TR_ONE) PA_GO(F_BINARY, TR_ONE, 8, false, 0);
-                PA_GO(F_BINARY, TR_ALL, 8, false, 0);
+                if (s.tr == TR_SCORE) PA_GO(F_BINARY, TR_SCORE, 8, 0);
+                if (s.tr == TR_ONE) PA_GO(F_BINARY, TR_ONE, 8, 0);
+                PA_GO(F_BINARY, TR_ALL, 8, 0);
             case F_DENSE:
-                if (s.tr == TR_SCORE) PA_GO(F_DENSE, TR_SCORE, 8, false, 0);
-                if (s.tr == TR_ONE) PA_GO(F_DENSE, TR_ONE, 8, false, 0);
-                PA_GO(F_DENSE, TR_ALL, 8, false, 0);
+                if (s.tr == TR_SCORE) PA_GO(F_DENSE, TR_SCORE, 8, 0);
+                if (s.tr == TR_ONE) PA_GO(F_DENSE, TR_ONE, 8, 0);
+                PA_GO(F_DENSE, TR_ALL, 8, 0);
             case F_DROWS:
-                if (s.tr == TR_SCORE) PA_GO(F_DROWS, TR_SCORE, 8, false, 0);
-                if (s.tr == TR_ONE) PA_GO(F_DROWS, TR_ONE, 8, false, 0);
-                PA_GO(F_DROWS, TR_ALL, 8, false, 0);
+                if (s.tr == TR_SCORE) PA_GO(F_DROWS, TR_SCORE, 8, 0);
+                if (s.tr == TR_ONE) PA_GO(F_DROWS, TR_ONE, 8, 0);
+                PA_GO(F_DROWS, TR_ALL, 8, 0);
             default: return hipErrorInvalidValue;
         }
     }
 #undef PA_GO
+#undef PA_GO_VAR
 }
 
 }  // namespace pa

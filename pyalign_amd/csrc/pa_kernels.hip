@@ -32,7 +32,7 @@ size_t long_lds_bytes(int form, int K1) {
 
 hipError_t launch_long(int loc, int dir, int gap, int form, int tr, bool fold_max, const KArgs &a,
                        const LongArgs &la, int grid, hipStream_t st) {
-    if (!long_supported(gap, form, tr) || la.n <= 0 || grid <= 0) return hipErrorInvalidValue;
+    if (!long_supported(gap, form, tr) || la.total_bands <= 0 || grid <= 0) return hipErrorInvalidValue;
     const size_t lds = long_lds_bytes(form, a.K1);
     const bool mx = dir == DIR_MAX;
     switch (loc) {
@@ -78,18 +78,8 @@ int band_R(int form, int tr) {
     return r4 ? 4 : 8;
 }
 
-bool supported_R(int form, int tr, bool fastmax, int R) {
-    if (form == F_TABLE && tr == TR_SCORE) {
-        if (fastmax) {
-            switch (R) {
-                case 1: case 2: case 3: case 4: case 5: case 6: case 7: case 8:
-                case 10: case 12: case 14: case 16: case 20: case 24: case 28: case 32:
-                    return true;
-                default: return false;
-            }
-        }
-        return R == 4 || R == 8 || R == 16 || R == 32;
-    }
+bool supported_R(int form, int tr, int R) {
+    if (form == F_TABLE && tr == TR_SCORE) return R == 4 || R == 8 || R == 16 || R == 32;
     return R == 8;
 }
 

@@ -53,11 +53,6 @@ constexpr int WAVE_LDS = 4 * TILE; // a wave's four blocks
 constexpr int MIN_LDS = 4 * B * KS;
 constexpr int PUSHES = 2;  // distances a wave pushes its four blocks to
 
-template <int DIR>
-__device__ __forceinline__ float opt(float a, float b) {
-    return DIR == DIR_MAX ? fmaxf(a, b) : fminf(a, b);
-}
-
 // lane r of a row of 16 <- lane r - M; lanes r < M read 0
 template <int M>
 __device__ __forceinline__ float row_shr0(float x) {
