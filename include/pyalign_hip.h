@@ -309,6 +309,9 @@ int pa_result_alignment(const pa_result *r, int64_t k, int32_t *s_to_t, int32_t 
  * path. */
 int pa_result_paths(const pa_result *r, int64_t *lens, int32_t *uv);
 int pa_result_alignments(const pa_result *r, int32_t *s_to_t, int32_t *t_to_s);
+/* The same in the solver's index type (int16 for index_bits 16, else int32),
+ * copied once: lens as in pa_result_paths; uv, s_to_t and t_to_s may be NULL. */
+int pa_result_solutions(const pa_result *r, int64_t *lens, void *uv, void *s_to_t, void *t_to_s);
 /* All-optimal iteration (TracebackIterators<true>, solver.h:1568-1743):
  * returns 1 and fills score/path for the next alignment of problem k, 0 at
  * the end.  The path is read with pa_result_iter_path afterwards. */

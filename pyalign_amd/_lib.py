@@ -91,6 +91,7 @@ SIGNATURES = {
     "pa_result_values": (ctypes.c_int, [_P, _I64, _P]),
     "pa_result_paths": (ctypes.c_int, [_P, _P, _P]),
     "pa_result_alignments": (ctypes.c_int, [_P, _P, _P]),
+    "pa_result_solutions": (ctypes.c_int, [_P, _P, _P, _P, _P]),
     "pa_result_traceback": (ctypes.c_int, [_P, _I64, _P]),
     "pa_result_edges_len": (_I64, [_P, _I64, _I32]),
     "pa_result_edges": (ctypes.c_int, [_P, _I64, _I32, _P]),

@@ -16,6 +16,7 @@
 #include <cstring>
 #include <limits>
 #include <memory>
+#include <mutex>
 #include <numeric>
 #include <set>
 #include <sstream>
@@ -132,6 +133,49 @@ struct pa_options {
 
 namespace {
 
+// Pinned host buffers of results, kept by a solver and its results: a
+// result's buffer is written by one device copy and goes back when the result
+// is freed (at most two wait for reuse).
+struct PinPool {
+    struct Buf {
+        char *p = nullptr;
+        size_t cap = 0;
+    };
+    std::mutex mu;
+    std::vector<Buf> idle;
+    ~PinPool() {
+        for (const Buf &b : idle) (void)hipHostFree(b.p);
+    }
+    Buf take(size_t bytes) {
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            for (size_t q = 0; q < idle.size(); q++) {
+                if (idle[q].cap < bytes) continue;
+                const Buf b = idle[q];
+                idle.erase(idle.begin() + std::ptrdiff_t(q));
+                return b;
+            }
+        }
+        Buf b;
+        b.cap = std::max<size_t>(bytes + bytes / 4, 4096);
+        HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&b.p), b.cap, hipHostMallocDefault));
+        return b;
+    }
+    void give(Buf b) {
+        if (!b.p) return;
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            idle.push_back(b);
+            if (idle.size() <= 2) return;
+            auto least = std::min_element(idle.begin(), idle.end(),
+                                          [](const Buf &x, const Buf &y) { return x.cap < y.cap; });
+            b = *least;
+            idle.erase(least);
+        }
+        (void)hipHostFree(b.p);
+    }
+};
+
 struct Plan {
     std::vector<Prob> probs;    // in group order
     std::vector<Group> groups;  // per launch, concatenated
@@ -180,7 +224,12 @@ struct pa_solver {
     int cus = 256;
     bool has_device = false;
     DevBuf b_border_s, b_border_t, b_probs, b_groups, b_queue, b_cs, b_ct, b_table, b_dense, b_rowbuf;
-    DevBuf b_scores, b_seeds, b_tb, b_path, b_path_off, b_path_len, b_dvals;
+    DevBuf b_scores, b_seeds, b_tb, b_path, b_off, b_path_len, b_dvals;
+    DevBuf b_out;  // a result's scores, lengths, alignments and paths, as they go to the host
+    std::shared_ptr<PinPool> pool = std::make_shared<PinPool>();
+    std::vector<int64_t> off;   // offsets of the last one-path result, and whether b_off holds them
+    bool off_uploaded = false;
+    std::vector<float> table;   // what b_table holds
     DevBuf b_progress, b_partials, b_band_err, b_band_probs;
     // general gap costs: w(k) * sgn for k = 0 .. lim (GeneralGapCostSolver's tensors)
     std::vector<float> ws_sgn, wt_sgn;
@@ -260,12 +309,24 @@ struct pa_result {
     int dir = 0, loc = 0, gap = 0, goal = 0;
     int index_bits = 16;
     bool remove_dup = true;
-    std::vector<float> scores;
     std::vector<int32_t> seeds;
     std::vector<int32_t> len_s, len_t;
-    // one-optimal paths
-    std::vector<int64_t> path_off;
-    std::vector<int32_t> path_len, paths;
+    // the device's results in one pinned buffer: scores and, one optimal path,
+    // path lengths, s_to_t, t_to_s and paths in the index type (problem k's
+    // from off[k], off[n + 1 + k] and off[2 (n + 1) + k] on: path points, s, t)
+    std::shared_ptr<PinPool> pool;
+    PinPool::Buf pin;
+    std::vector<int64_t> off;
+    const float *scores = nullptr;
+    const int32_t *path_len = nullptr;
+    const char *s_to_t = nullptr, *t_to_s = nullptr, *paths = nullptr;
+    ~pa_result() {
+        if (pool) pool->give(pin);
+    }
+    int width() const { return index_bits == 16 ? 2 : 4; }
+    int64_t path_at(int64_t k) const { return off[size_t(k)]; }
+    int64_t s_at(int64_t k) const { return off[size_t(n + 1 + k)]; }
+    int64_t t_at(int64_t k) const { return off[size_t(2 * (n + 1) + k)]; }
     // all-optimal: traceback bits and local D values; Solution matrices:
     // the traceback bits and every layer's values, plus the borders
     std::vector<uint32_t> tb;
@@ -1052,6 +1113,70 @@ void stage_payload(pa_solver &s, const Input &in, hipStream_t st, const void *&c
 }
 
 
+// The offsets of every problem's path points (len_s + len_t + 2 of them),
+// s and t symbols in concatenated outputs, on the host and the device (both
+// kept while lengths repeat).
+void place_results(pa_solver &s, const Input &in, hipStream_t st, pa_result &r) {
+    const size_t n1 = size_t(in.n) + 1;
+    r.off.resize(3 * n1);
+    int64_t p = 0, a = 0, b = 0;
+    for (size_t k = 0; k < n1; k++) {
+        r.off[k] = p;
+        r.off[n1 + k] = a;
+        r.off[2 * n1 + k] = b;
+        if (k == size_t(in.n)) break;
+        p += int64_t(in.len_s[k]) + in.len_t[k] + 2;
+        a += in.len_s[k];
+        b += in.len_t[k];
+    }
+    if (!s.off_uploaded || s.off != r.off) {
+        s.off_uploaded = false;
+        s.off = r.off;
+        upload(st, s.b_off, s.off.data(), s.off.size());
+        s.off_uploaded = true;
+    }
+    s.b_path.ensure(size_t(std::max<int64_t>(p, 1)) * 8);
+    s.b_path_len.ensure(size_t(std::max<int64_t>(in.n, 1)) * 4);
+}
+
+// A result's scores and, with paths, its packed paths and alignments, on
+// their way to its pinned buffer (one copy; the caller waits for the stream).
+void fetch_results(pa_solver &s, hipStream_t st, pa_result &r, const float *scores, bool paths) {
+    const size_t n = size_t(r.n);
+    if (!n) return;
+    auto pad = [](size_t x) { return (x + 15) / 16 * 16; };
+    const size_t w = size_t(r.width());
+    const size_t at_len = pad(n * 4), at_s = at_len + pad(n * 4);
+    const size_t at_t = paths ? at_s + pad(size_t(r.s_at(r.n)) * w) : 0;
+    const size_t at_p = paths ? at_t + pad(size_t(r.t_at(r.n)) * w) : 0;
+    const size_t bytes = paths ? at_p + size_t(r.path_at(r.n)) * 2 * w : n * 4;
+    r.pool = s.pool;
+    r.pin = r.pool->take(bytes);
+    const void *src = scores;
+    if (paths) {
+        s.b_out.ensure(bytes);
+        char *o = s.b_out.as<char>();
+        HIPCHK(launch_pack(r.width(), r.n, s.b_path.as<int32_t>(), s.b_off.as<int64_t>(), s.b_path_len.as<int32_t>(),
+                           scores, reinterpret_cast<float *>(o), reinterpret_cast<int32_t *>(o + at_len), o + at_s,
+                           o + at_t, o + at_p, st));
+        src = o;
+        r.path_len = reinterpret_cast<const int32_t *>(r.pin.p + at_len);
+        r.s_to_t = r.pin.p + at_s;
+        r.t_to_s = r.pin.p + at_t;
+        r.paths = r.pin.p + at_p;
+    }
+    r.scores = reinterpret_cast<const float *>(r.pin.p);
+    HIPCHK(hipMemcpyAsync(r.pin.p, src, bytes, hipMemcpyDeviceToHost, st));
+}
+
+// The table on the device (kept while it repeats).
+void stage_table(pa_solver &s, const Input &in, hipStream_t st) {
+    if (in.table == s.table && s.b_table.p) return;
+    s.table.clear();
+    upload(st, s.b_table, in.table.data(), in.table.size());
+    s.table = in.table;
+}
+
 // Whether a general-gap solve's folds return the strict folds' bits in any
 // order: similarities and costs finite (sums cannot overflow) or, for
 // similarities, the worst value, and no candidate -0 (a sum is -0 only where
@@ -1190,7 +1315,7 @@ void run_wsb(pa_solver &s, const Input &in, const Job &job, std::unique_ptr<pa_r
     const void *codes_s = nullptr, *codes_t = nullptr;
     const float *dense = nullptr;
     stage_payload(s, in, st, codes_s, codes_t, dense);
-    if (job.form == F_TABLE || job.form == F_TABLE_G) upload(st, s.b_table, in.table.data(), in.table.size());
+    if (job.form == F_TABLE || job.form == F_TABLE_G) stage_table(s, in, st);
     s.b_dvals.ensure(size_t(std::max<int64_t>(words, 1)) * 4);
     float *scores = scores_device;
     if (!scores) {
@@ -1223,15 +1348,10 @@ void run_wsb(pa_solver &s, const Input &in, const Job &job, std::unique_ptr<pa_r
     if (result) {
         r = std::make_unique<pa_result>();
         if (job.tr == TR_ONE) {
-            r->path_off.resize(size_t(n) + 1);
-            r->path_off[0] = 0;
-            for (int64_t k = 0; k < n; k++)
-                r->path_off[size_t(k) + 1] = r->path_off[size_t(k)] + in.len_s[k] + in.len_t[k] + 2;
-            upload(st, s.b_path_off, r->path_off.data(), r->path_off.size());
-            s.b_path.ensure(size_t(std::max<int64_t>(r->path_off.back(), 1)) * 8);
-            s.b_path_len.ensure(size_t(std::max<int64_t>(n, 1)) * 4);
+            r->n = n;
+            place_results(s, in, st, *r);
             path = s.b_path.as<int32_t>();
-            path_off = s.b_path_off.as<int64_t>();
+            path_off = s.b_off.as<int64_t>();
             path_len = s.b_path_len.as<int32_t>();
         }
     }
@@ -1272,17 +1392,9 @@ void run_wsb(pa_solver &s, const Input &in, const Job &job, std::unique_ptr<pa_r
     r->remove_dup = o.remove_dup;
     r->len_s.assign(in.len_s, in.len_s + n);
     r->len_t.assign(in.len_t, in.len_t + n);
-    r->scores.resize(size_t(n));
-    r->seeds.resize(size_t(n) * 2);
-    if (job.tr == TR_ONE) {
-        r->path_len.resize(size_t(n));
-        r->paths.resize(size_t(r->path_off.back()) * 2);
-        HIPCHK(hipMemcpyAsync(r->path_len.data(), path_len, size_t(n) * 4, hipMemcpyDeviceToHost, st));
-        if (!r->paths.empty())
-            HIPCHK(hipMemcpyAsync(r->paths.data(), path, r->paths.size() * 4, hipMemcpyDeviceToHost, st));
-    }
-    if (n) {
-        HIPCHK(hipMemcpyAsync(r->scores.data(), scores, size_t(n) * 4, hipMemcpyDeviceToHost, st));
+    fetch_results(s, st, *r, scores, job.tr == TR_ONE);
+    if (job.tr == TR_ALL && n) {
+        r->seeds.resize(size_t(n) * 2);
         HIPCHK(hipMemcpyAsync(r->seeds.data(), a.seeds, size_t(n) * 8, hipMemcpyDeviceToHost, st));
     }
     r->matrices = in.matrices;
@@ -1566,7 +1678,7 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
     const void *codes_s = nullptr, *codes_t = nullptr;
     const float *dense = nullptr;
     stage_payload(s, in, st, codes_s, codes_t, dense);
-    if (job.form == F_TABLE || job.form == F_TABLE_G) upload(st, s.b_table, in.table.data(), in.table.size());
+    if (job.form == F_TABLE || job.form == F_TABLE_G) stage_table(s, in, st);
     s.b_rowbuf.ensure(size_t(std::max<int64_t>(plan.rowbuf, 1)) * sizeof(float2));
     float *scores = scores_device;
     if (!scores) {
@@ -1785,23 +1897,13 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
     r->remove_dup = o.remove_dup;
     r->len_s.assign(in.len_s, in.len_s + n);
     r->len_t.assign(in.len_t, in.len_t + n);
-    r->scores.resize(static_cast<size_t>(n));
     if (job.tr == TR_ONE) {
-        r->path_off.resize(size_t(n) + 1);
-        r->path_off[0] = 0;
-        for (int64_t k = 0; k < n; k++) r->path_off[size_t(k) + 1] = r->path_off[size_t(k)] + in.len_s[k] + in.len_t[k] + 2;
-        upload(st, s.b_path_off, r->path_off.data(), r->path_off.size());
-        s.b_path.ensure(size_t(std::max<int64_t>(r->path_off.back(), 1)) * 8);
-        s.b_path_len.ensure(size_t(std::max<int64_t>(n, 1)) * 4);
+        place_results(s, in, st, *r);
         HIPCHK(launch_walk(job.gap, s.b_probs.as<Prob>(), int64_t(plan.probs.size()), s.b_tb.as<uint32_t>(), seeds,
-                           s.b_path.as<int32_t>(), s.b_path_off.as<int64_t>(), s.b_path_len.as<int32_t>(), st));
-        r->path_len.resize(static_cast<size_t>(n));
-        r->paths.resize(size_t(r->path_off.back()) * 2);
-        HIPCHK(hipMemcpyAsync(r->path_len.data(), s.b_path_len.p, size_t(n) * 4, hipMemcpyDeviceToHost, st));
-        if (!r->paths.empty())
-            HIPCHK(hipMemcpyAsync(r->paths.data(), s.b_path.p, r->paths.size() * 4, hipMemcpyDeviceToHost, st));
+                           s.b_path.as<int32_t>(), s.b_off.as<int64_t>(), s.b_path_len.as<int32_t>(), st));
     }
-    if (job.tr != TR_SCORE) {
+    fetch_results(s, st, *r, scores, job.tr == TR_ONE);
+    if (job.tr == TR_ALL) {
         r->seeds.resize(size_t(n) * 2);
         HIPCHK(hipMemcpyAsync(r->seeds.data(), seeds, size_t(n) * 8, hipMemcpyDeviceToHost, st));
     }
@@ -1823,7 +1925,6 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
         for (const Prob &pr : plan.probs) r->probs[size_t(pr.out)] = pr;
         if (job.tr == TR_ALL) r->iters.resize(static_cast<size_t>(n));
     }
-    if (n) HIPCHK(hipMemcpyAsync(r->scores.data(), scores, size_t(n) * 4, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     check_band(s);
     float ms = 0.0f;
@@ -2894,7 +2995,7 @@ int64_t pa_result_count(const pa_result *r) { return r ? r->n : 0; }
 int pa_result_scores(const pa_result *r, float *out) {
     return guard([&] {
         if (!r || !out) fail(PA_EINVAL, "null argument");
-        std::copy(r->scores.begin(), r->scores.end(), out);
+        if (r->n) std::memcpy(out, r->scores, size_t(r->n) * 4);
     });
 }
 
@@ -2909,12 +3010,22 @@ int64_t pa_result_path_len(const pa_result *r, int64_t k) {
     return r->path_len[size_t(k)];
 }
 
+// `count` values of the result's index type at p + at, as int32
+static void widen(const pa_result *r, const char *p, int64_t at, int64_t count, int32_t *out) {
+    if (r->width() == 4) {
+        std::memcpy(out, p + at * 4, size_t(count) * 4);
+    } else {
+        const int16_t *v = reinterpret_cast<const int16_t *>(p) + at;
+        for (int64_t q = 0; q < count; q++) out[q] = v[q];
+    }
+}
+
 int pa_result_path(const pa_result *r, int64_t k, int32_t *uv) {
     return guard([&] {
         if (!r || !uv || k < 0 || k >= r->n || r->goal != PA_GOAL_ONE) fail(PA_EINVAL, "no path for this problem");
         const int32_t m = r->path_len[size_t(k)];
         if (m < 0) fail(PA_EINVAL, "no path for this problem");
-        std::memcpy(uv, r->paths.data() + 2 * r->path_off[size_t(k)], size_t(m) * 8);
+        widen(r, r->paths, 2 * r->path_at(k), 2 * int64_t(m), uv);
     });
 }
 
@@ -2926,9 +3037,26 @@ int pa_result_paths(const pa_result *r, int64_t *lens, int32_t *uv) {
             const int32_t m = r->path_len[size_t(k)];
             lens[k] = m;
             if (m <= 0) continue;
-            if (uv) std::memcpy(uv + 2 * at, r->paths.data() + 2 * r->path_off[size_t(k)], size_t(m) * 8);
+            if (uv) widen(r, r->paths, 2 * r->path_at(k), 2 * int64_t(m), uv + 2 * at);
             at += m;
         }
+    });
+}
+
+int pa_result_solutions(const pa_result *r, int64_t *lens, void *uv, void *s_to_t, void *t_to_s) {
+    return guard([&] {
+        if (!r || !lens || r->goal != PA_GOAL_ONE) fail(PA_EINVAL, "not a one-optimal result");
+        const size_t w = size_t(r->width());
+        char *out = static_cast<char *>(uv);
+        for (int64_t k = 0; k < r->n; k++) {
+            const int32_t m = r->path_len[size_t(k)];
+            lens[k] = m;
+            if (m <= 0 || !out) continue;
+            std::memcpy(out, r->paths + size_t(r->path_at(k)) * 2 * w, size_t(m) * 2 * w);
+            out += size_t(m) * 2 * w;
+        }
+        if (s_to_t && r->n) std::memcpy(s_to_t, r->s_to_t, size_t(r->s_at(r->n)) * w);
+        if (t_to_s && r->n) std::memcpy(t_to_s, r->t_to_s, size_t(r->t_at(r->n)) * w);
     });
 }
 
@@ -2962,20 +3090,9 @@ static void alignment_from_path(const int32_t *uv, int64_t m, int32_t ls, int32_
 int pa_result_alignments(const pa_result *r, int32_t *s_to_t, int32_t *t_to_s) {
     return guard([&] {
         if (!r || !s_to_t || !t_to_s || r->goal != PA_GOAL_ONE) fail(PA_EINVAL, "not a one-optimal result");
-        int64_t as = 0, at = 0;
-        for (int64_t k = 0; k < r->n; k++) {
-            const int32_t ls = r->len_s[size_t(k)], lt = r->len_t[size_t(k)];
-            const int32_t m = r->path_len[size_t(k)];
-            if (m < 0) {
-                std::fill(s_to_t + as, s_to_t + as + ls, -1);
-                std::fill(t_to_s + at, t_to_s + at + lt, -1);
-            } else {
-                alignment_from_path(r->paths.data() + 2 * r->path_off[size_t(k)], m, ls, lt, s_to_t + as,
-                                    t_to_s + at);
-            }
-            as += ls;
-            at += lt;
-        }
+        if (!r->n) return;
+        widen(r, r->s_to_t, 0, r->s_at(r->n), s_to_t);
+        widen(r, r->t_to_s, 0, r->t_at(r->n), t_to_s);
     });
 }
 
@@ -2984,13 +3101,8 @@ int pa_result_alignment(const pa_result *r, int64_t k, int32_t *s_to_t, int32_t 
         if (!r || k < 0 || k >= r->n) fail(PA_EINVAL, "bad problem index");
         const int32_t ls = r->len_s[size_t(k)], lt = r->len_t[size_t(k)];
         if (r->goal == PA_GOAL_ONE) {
-            const int32_t m = r->path_len[size_t(k)];
-            if (m < 0) {
-                std::fill(s_to_t, s_to_t + ls, -1);
-                std::fill(t_to_s, t_to_s + lt, -1);
-                return;
-            }
-            alignment_from_path(r->paths.data() + 2 * r->path_off[size_t(k)], m, ls, lt, s_to_t, t_to_s);
+            widen(r, r->s_to_t, r->s_at(k), ls, s_to_t);
+            widen(r, r->t_to_s, r->t_at(k), lt, t_to_s);
         } else if (r->goal == PA_GOAL_ALL) {
             const IterState *it = r->iters[size_t(k)].get();
             if (!it || it->cur_path.empty()) fail(PA_EINVAL, "no current alignment");

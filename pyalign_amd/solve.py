@@ -30,11 +30,14 @@ from .problems.factory import AlphabetEncoder, AlphabetProblem, SeriesProblem
 class Solution:
     """The optimal solution of one problem: score, alignment, path."""
 
+    # (a bag makes thousands: no dict unless values or an attribute need it)
+    __slots__ = ("_problem", "_solver", "_solution", "_alignment", "_traceback", "__dict__", "__weakref__")
+
     def __init__(self, problem, solver, solution):
         self._problem = problem
         self._solver = solver
         self._solution = solution
-        self._traceback = {}
+        self._alignment = self._traceback = None  # made on first use
 
     @property
     def problem(self):
@@ -44,11 +47,15 @@ class Solution:
     def score(self):
         return self._solution.score
 
-    @cached_property
+    @property
     def alignment(self):
-        if self._solution.alignment is None:
-            return None
-        return Alignment(self._problem, self._solver, self._solution.alignment)
+        if self._alignment is None:
+            core = self._solution
+            if not isinstance(core, algorithm._BagSolution):  # (one reads like its own alignment)
+                core = core.alignment
+            if core is not None:
+                self._alignment = Alignment(self._problem, self._solver, core)
+        return self._alignment
 
     @property
     def shape(self):
@@ -59,6 +66,8 @@ class Solution:
         return self._solution.values
 
     def traceback(self, form="matrix"):
+        if self._traceback is None:
+            self._traceback = {}
         if form not in self._traceback:
             if form == "matrix":
                 self._traceback[form] = self._solution.traceback_as_matrix
@@ -68,7 +77,7 @@ class Solution:
                 return ValueError(form)
         return self._traceback[form]
 
-    @cached_property
+    @property
     def path(self):
         return self._solution.path
 
@@ -79,6 +88,8 @@ class Solution:
 
 class Alignment:
     """A specific alignment that is part of a solution."""
+
+    __slots__ = ("_problem", "_solver", "_alignment", "__dict__", "__weakref__")
 
     def __init__(self, problem, solver, alignment):
         self._problem = problem
