@@ -1016,7 +1016,8 @@ struct Input {
 };
 
 // Whether max / min folds (and traceback codes from equality tests) keep the
-// strict folds' bits in alignments over a table or binary symbols:
+// strict folds' bits in alignments over a table, binary symbols or a dense
+// matrix:
 // similarities finite (or the pad's worst value) and never -0, and, for
 // maximising global problems, gap costs above zero (borders below -0), so that
 // no candidate is -0 or NaN.
@@ -1025,6 +1026,7 @@ bool folds_max(const pa_solver &s, const Input &in, const Job &job) {
     auto exact = [](float x) { return std::isfinite(x) && !(x == 0.0f && std::signbit(x)); };
     if (job.loc == LOC_GLOBAL && job.dir == DIR_MAX && !(s.go_s < 0.0f && s.go_t < 0.0f)) return false;
     if (job.form == F_BINARY) return exact(in.eq) && exact(in.ne);
+    if (job.form == F_DENSE) return true;  // (the kernel looks at the values and falls back)
     if (job.form != F_TABLE) return false;
     const float w = worst(s.opt.dir);
     return std::all_of(in.table.begin(), in.table.end(), [&](float x) { return exact(x) || x == w; });

@@ -28,8 +28,8 @@ constexpr size_t DROWS_LDS = size_t(256) * DROWS_LANE_FLOATS * 4;
 // (2 bits linear/DTW, 4 bits affine) or the full tie set (8 bits per cell).
 enum { TR_SCORE = 0, TR_ONE = 1, TR_ALL = 2 };
 // Builds of the general kernel that keeps a traceback: the usual one, one that
-// also stores cell values (KArgs::dvals), and alignments over a table or
-// binary symbols with max / min folds.
+// also stores cell values (KArgs::dvals), and alignments over a table, binary
+// symbols or a dense matrix with max / min folds.
 enum { VAR_PLAIN = 0, VAR_VALUES = 1, VAR_MAX = 2 };
 
 constexpr int WAVE = 64;

@@ -43,6 +43,21 @@ __device__ __forceinline__ float opt(float a, float b) {
     return DIR == DIR_MAX ? fmaxf(a, b) : fminf(a, b);
 }
 
+// Traceback flags without lane masks: the sign of lead(a, b) says that b is
+// strictly better than a (their difference is exact in sign; equal values,
+// infinities too, give +0 or a positive NaN), and push_sign shifts it into a
+// word with one v_alignbit_b32.  A compare, its 64-bit mask in scalar
+// registers and a select of a constant cost as many instructions and the wait
+// states between mask and select (38 s_nop in an 8-cell Gotoh step; 2,048 local
+// pairs, the general kernel's part: 1.43 -> 1.19 ms).
+template <int DIR>
+__device__ __forceinline__ float lead(float a, float b) {
+    return DIR == DIR_MAX ? a - b : b - a;
+}
+__device__ __forceinline__ uint32_t push_sign(uint32_t word, float x) {
+    return __builtin_amdgcn_alignbit(word, __float_as_uint(x), 31);
+}
+
 // lane k <- lane k-1 (wave_shr:1); lane 0 keeps its own value
 __device__ __forceinline__ float shr1(float x) {
     return __int_as_float(
@@ -93,8 +108,10 @@ __device__ __forceinline__ void band_wait(const KArgs &a, int idx, uint32_t need
 
 extern __shared__ float pa_dyn_lds[];  // the launch's dynamic LDS (table or staging windows)
 
+// Returns whether the group's results stand: false where a dense similarity
+// met by max / min folds is infinite, NaN or -0, which only strict folds take.
 template <int LOC, int DIR, int GAP, int FORM, int TR, int R, int SD, int VAR, bool BAND = false>
-__device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, const float *__restrict__ tab,
+__device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, const float *__restrict__ tab,
                                             int lane) {
     constexpr float W = worst<DIR>();
     constexpr bool DENSE = FORM == F_DENSE || FORM == F_DROWS;
@@ -133,6 +150,7 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
     float rbest = W, cbest = W;
     int rj = -1, ci = -1;
     float gscore = W;
+    [[maybe_unused]] bool odd_value = false;
     // steady steps: the members' shortest length and fewest strips
     int min_lt = has ? lt : 0x7fffffff, min_nst = has ? nst : 0x7fffffff;
     for (int m = 1; m < WAVE; m <<= 1) {
@@ -392,6 +410,22 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
             if (STEADY || (act && j >= 0 && j < lt)) {
                 float Dd = Ddiag, Dup = inD, Pup = inP;
                 uint32_t tbw[WPC];
+                // max / min folds: the codes as signs, pushed first cell first
+                constexpr bool CODES = MXF && TR == TR_ONE && !NOTB;
+                static_assert(!CODES || BITS * R <= 32, "one word of signs a step");
+                [[maybe_unused]] uint32_t signs = 0;
+                // (the code's low bit is made of two flags once the step's cells are done; a
+                // local cell's code is 0 where its value is not above zero)
+                [[maybe_unused]] auto push_code = [&](float not_diag, float not_up, float D) {
+                    uint32_t b0 = __float_as_uint(not_up), b1 = __float_as_uint(not_diag);
+                    if constexpr (LOC == LOC_LOCAL && GAP != GAP_DTW) {
+                        const uint32_t above = __float_as_uint(lead<DIR>(0.0f, D));
+                        b0 = above & (~b1 | b0);
+                        b1 &= above;
+                    }
+                    signs = push_sign(signs, __uint_as_float(b0));
+                    signs = push_sign(signs, __uint_as_float(b1));
+                };
 #pragma unroll
                 for (int w = 0; w < WPC; ++w) tbw[w] = 0;
 
@@ -415,6 +449,8 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
                         if constexpr (PADW) S = rv[r] ? S : W;
                     } else if constexpr (DENSE) {
                         S = PADW ? (rv[r] ? Scol[r] : W) : Scol[r];
+                        // NaN, infinities, -0 (in padded rows as well: their loads read valid memory)
+                        if constexpr (VAR == VAR_MAX) odd_value |= __builtin_amdgcn_classf(Scol[r], 0x227);
                     } else {
                         // squared Euclidean cost, dimensions summed in order
                         float c = 0.0f;
@@ -438,7 +474,7 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
                             const float m = DIR == DIR_MAX ? fmaxf(fmaxf(Dd, Dup), Din[r])
                                                            : fminf(fminf(Dd, Dup), Din[r]);
                             D = m + S;
-                            bits = Dd == m ? 1u : (Dup == m ? 2u : 3u);
+                            if constexpr (CODES) push_code(lead<DIR>(Dd, m), lead<DIR>(Dup, m), D);
                         } else {
                             float m = Dd;
                             int src = 1;
@@ -454,8 +490,7 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
                         const float lf = Din[r] + go_t;
                         if constexpr (MXF) {
                             D = opt<DIR>(opt<DIR>(LOC == LOC_LOCAL ? opt<DIR>(dg, 0.0f) : dg, up), lf);
-                            bits = dg == D ? 1u : (up == D ? 2u : 3u);
-                            if constexpr (LOC == LOC_LOCAL) bits = D == 0.0f ? 0u : bits;
+                            if constexpr (CODES) push_code(lead<DIR>(dg, D), lead<DIR>(up, D), D);
                         } else {
                             int src;
                             if constexpr (LOC == LOC_LOCAL) {
@@ -482,9 +517,11 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
                             P = opt<DIR>(po, pe);
                             Q = opt<DIR>(qo, qe);
                             D = opt<DIR>(opt<DIR>(LOC == LOC_LOCAL ? opt<DIR>(dg, 0.0f) : dg, P), Q);
-                            bits = dg == D ? 1u : (P == D ? 2u : 3u);
-                            if constexpr (LOC == LOC_LOCAL) bits = D == 0.0f ? 0u : bits;
-                            bits |= (better<DIR>(pe, po) ? 4u : 0u) | (better<DIR>(qe, qo) ? 8u : 0u);
+                            if constexpr (CODES) {
+                                push_code(lead<DIR>(dg, D), lead<DIR>(P, D), D);
+                                signs = push_sign(signs, lead<DIR>(po, pe));  // P extends
+                                signs = push_sign(signs, lead<DIR>(qo, qe));  // Q extends
+                            }
                         } else {
                             const bool pext = better<DIR>(pe, po);
                             P = pext ? pe : po;
@@ -542,7 +579,7 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
                             }
                         }
                     }
-                    if constexpr (TR != TR_SCORE && !NOTB) tbw[(r * BITS) / 32] |= bits << ((r * BITS) % 32);
+                    if constexpr (TR != TR_SCORE && !NOTB && !CODES) tbw[(r * BITS) / 32] |= bits << ((r * BITS) % 32);
 
                     Dd = Din[r];
                     Dout[r] = D;
@@ -561,6 +598,14 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
                     }
                 }
 
+                if constexpr (CODES) {
+                    // the first cell's flags to the lowest bits; then, not
+                    // local: low bit = the diagonal chosen, or P (up) not
+                    constexpr int UNUSED = BITS > 0 && BITS * R <= 32 ? 32 - BITS * R : 0;
+                    constexpr uint32_t LOW = (BITS == 4 ? 0x11111111u : 0x55555555u) >> UNUSED;
+                    tbw[0] = __builtin_bitreverse32(signs) >> UNUSED;
+                    if constexpr (LOC != LOC_LOCAL || GAP == GAP_DTW) tbw[0] |= ~(tbw[0] >> 1) & LOW;
+                }
                 if constexpr (TR != TR_SCORE && !NOTB) {
                     // problems of a checkpointed forward keep no traceback
                     if (pr.tb_off != NO_TB_OFF) {
@@ -660,6 +705,9 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
         };
         if constexpr (VAR == VAR_VALUES) {
             sweep(integral_constant<int, 1>{});
+        } else if constexpr (VAR == VAR_MAX && DENSE) {
+            if (a.probs[g.first].tb_off == NO_TB_OFF) sweep(integral_constant<int, 4>{});
+            else sweep(integral_constant<int, 3>{});
         } else if constexpr (VAR == VAR_MAX) {
             sweep(integral_constant<int, 3>{});
         } else if constexpr (TR == TR_ONE) {
@@ -752,7 +800,7 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
             bp.pad = 0;
             a.partials[pr.band + g.strip] = bp;
         }
-        return;
+        return true;
     }
     if (has && l == 0) {
         if (ls == 0 || lt == 0) {
@@ -766,6 +814,7 @@ __device__ __forceinline__ void solve_group(const KArgs &a, const Group &g, cons
             }
         }
     }
+    return !(VAR == VAR_MAX && DENSE) || !__any(odd_value);
 }
 
 // ---------------------------------------------------------------------------
@@ -1151,13 +1200,18 @@ __global__ __launch_bounds__(256) void pa_solve_kernel(KArgs a) {
     // leaves once its ticket passes the group count.
     for (uint32_t t = first_ticket(a); t < uint32_t(a.n_groups); t = next_ticket(a, lane)) {
         const Group &g = a.groups[t];
+        constexpr bool DENSE_MAX = VAR == VAR_MAX && (FORM == F_DENSE || FORM == F_DROWS);
         if constexpr (TR != TR_ALL) {
             if (g.strip >= 0) {
-                solve_group<LOC, DIR, GAP, FORM, TR, R, SD, VAR, true>(a, g, tab, lane);
+                solve_group<LOC, DIR, GAP, FORM, TR, R, SD, DENSE_MAX ? VAR_PLAIN : VAR, true>(a, g, tab, lane);
                 continue;
             }
         }
-        solve_group<LOC, DIR, GAP, FORM, TR, R, SD, VAR>(a, g, tab, lane);
+        // dense similarities are not known beforehand: max / min folds that
+        // watch for values they cannot take, and strict folds after those
+        if (!solve_group<LOC, DIR, GAP, FORM, TR, R, SD, VAR>(a, g, tab, lane)) {
+            if constexpr (DENSE_MAX) solve_group<LOC, DIR, GAP, FORM, TR, R, SD, VAR_PLAIN>(a, g, tab, lane);
+        }
     }
 }
 
@@ -1194,7 +1248,7 @@ static hipError_t dispatch_lg(const LaunchSpec &s, const KArgs &a, hipStream_t s
     do {                                                                                         \
         if constexpr (TR != TR_SCORE)                                                            \
             if (s.var == VAR_VALUES) PA_GO_VAR(FORM, TR, R, SD, VAR_VALUES);                     \
-        if constexpr (TR == TR_ONE && GAP != GAP_DTW && (FORM == F_TABLE || FORM == F_BINARY))   \
+        if constexpr (TR == TR_ONE && GAP != GAP_DTW && FORM != F_TABLE_G && FORM != F_SERIES)   \
             if (s.var == VAR_MAX) PA_GO_VAR(FORM, TR, R, SD, VAR_MAX);                           \
         PA_GO_VAR(FORM, TR, R, SD, VAR_PLAIN);                                                   \
     } while (0)

@@ -39,6 +39,7 @@ def test_table_folds(loc, gap, direction, n):
     table[table == 0] = 0.0  # (no -0 left by the symmetrisation)
     if direction == "minimize":
         table = np.where(table == 0, 0.0, -table).astype(np.float32)
+    table[0, 1] = -np.inf if direction == "maximize" else np.inf  # (a pair that never matches)
     strict = table.copy()
     strict[5, 5] = -0.0
     payload = dict(codes_s=cs, codes_t=ct, off_s=os_, off_t=ot)
@@ -53,6 +54,40 @@ def test_table_folds(loc, gap, direction, n):
             if a[k].score is not None:
                 assert np.float32(a[k].score).tobytes() == np.float32(b[k].score).tobytes(), k
                 assert np.array_equal(a[k].path, b[k].path), (k, ls[k], lt[k])
+
+
+@pytest.mark.parametrize("loc", list(LOCS))
+@pytest.mark.parametrize("direction", ["maximize", "minimize"])
+@pytest.mark.parametrize("odd", [None, "worst", "-0", "inf", "nan"])
+def test_dense_folds(loc, direction, odd):
+    """Dense similarities: codes from signs, and strict folds again for the
+    groups that meet a value max / min folds cannot take."""
+    rng = np.random.default_rng(3 + len(loc))
+    n = 60
+    ls, lt = lengths(rng, n, 1, 90, 8, 90)
+    ls[:3], lt[:3] = (600, 513, 64), (40, 33, 500)
+    flat = rng.integers(-2, 3, int((ls.astype(np.int64) * lt).sum())).astype(np.float32)
+    flat[flat == 0] = 0.0
+    off = np.concatenate([[0], np.cumsum(ls.astype(np.int64) * lt)[:-1]])
+    if odd:
+        bad = {"worst": -np.inf if direction == "maximize" else np.inf, "-0": -0.0,
+               "inf": np.inf if direction == "maximize" else -np.inf, "nan": np.nan}[odd]
+        for k in (0, 5, 17):
+            flat[off[k] + rng.integers(0, ls[k] * lt[k], 3)] = bad
+        flat[off[9]] = bad  # the first cell: -0 beside the border's -0
+    odir = O.MAXIMIZE if direction == "maximize" else O.MINIMIZE
+    for gap in GAPS:
+        got = make_solver(loc, gap, direction, pa.Solution, 1024, 1024).solve_ragged("solution", "dense", ls, lt,
+                                                                                   dense=flat, dense_off=off)
+        for k in range(n):
+            S = flat[off[k]:off[k] + ls[k] * lt[k]].reshape(ls[k], lt[k])
+            ref = O.OracleResult(O.make_config(locality=LOCS[loc][1], direction=odir, gap=gap, goal=O.GOAL_ONE,
+                                               lim_s=1024, lim_t=1024), S)
+            if not ref.has_seed:
+                assert got[k].score is None, k
+                continue
+            assert np.float32(got[k].score).tobytes() == ref.score.tobytes(), (k, gap)
+            assert np.array_equal(np.asarray(got[k].path, np.int32), ref.path()), (k, gap)
 
 
 @pytest.mark.parametrize("loc", list(LOCS))
