@@ -197,7 +197,8 @@ struct Plan {
 // planning and the descriptor upload.
 struct PlanCache {
     bool valid = false;
-    bool uploaded = false;  // b_probs / b_groups / b_band_probs hold this plan
+    bool uploaded = false;  // b_probs holds this plan: descriptors, groups and band words
+    size_t groups_at = 0, bands_at = 0;  // bytes into b_probs
     std::vector<int64_t> key;
     std::vector<int32_t> len_s, len_t;
     std::vector<int64_t> off_s, off_t;
@@ -223,14 +224,14 @@ struct pa_solver {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int cus = 256;
     bool has_device = false;
-    DevBuf b_border_s, b_border_t, b_probs, b_groups, b_queue, b_cs, b_ct, b_table, b_dense, b_rowbuf;
+    DevBuf b_border_s, b_border_t, b_probs, b_queue, b_cs, b_ct, b_table, b_dense, b_rowbuf;
     DevBuf b_scores, b_seeds, b_tb, b_path, b_off, b_path_len, b_dvals;
     DevBuf b_out;  // a result's scores, lengths, alignments and paths, as they go to the host
     std::shared_ptr<PinPool> pool = std::make_shared<PinPool>();
     std::vector<int64_t> off;   // offsets of the last one-path result, and whether b_off holds them
     bool off_uploaded = false;
     std::vector<float> table;   // what b_table holds
-    DevBuf b_progress, b_partials, b_band_err, b_band_probs;
+    DevBuf b_progress, b_partials, b_band_err;
     // general gap costs: w(k) * sgn for k = 0 .. lim (GeneralGapCostSolver's tensors)
     std::vector<float> ws_sgn, wt_sgn;
     bool gen_ready = false;
@@ -585,7 +586,7 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
     // an eighth of a SIMD's share of the work for the fast kernel, a
     // sixteenth for the general kernel (both measured best)
     // (of a large bag every few problems stand for all)
-    const int64_t stride = std::max<int64_t>(1, n / 4096);
+    const int64_t stride = std::max<int64_t>(1, n / 1024);
     double total = 0.0;
     for (int64_t k = 0; k < n; k += stride) {
         if (ls[k] <= 0 || lt[k] <= 0) continue;
@@ -1646,9 +1647,14 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
     }
     if (!pc.uploaded) {
         const Plan &pl = pc.plan;
+        // descriptors, groups and band words in one buffer and one copy (three
+        // copies cost a training step about 40 us of an idle GPU)
         const size_t nb[3] = {pl.probs.size() * sizeof(Prob), pl.groups.size() * sizeof(Group),
                               pl.band_words.size() * sizeof(int32_t)};
-        const size_t al = 256, total = (nb[0] + al) + (nb[1] + al) + (nb[2] + al);
+        const size_t al = 256;
+        pc.groups_at = (nb[0] + al - 1) / al * al;
+        pc.bands_at = pc.groups_at + (nb[1] + al - 1) / al * al;
+        const size_t total = pc.bands_at + nb[2];
         if (s.stage_pending) HIPCHK(hipEventSynchronize(s.stage_ev));
         s.stage_pending = false;
         if (s.stage_cap < total) {
@@ -1658,16 +1664,11 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
             HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&s.stage), total + total / 4, hipHostMallocDefault));
             s.stage_cap = total + total / 4;
         }
-        const void *src[3] = {pl.probs.data(), pl.groups.data(), pl.band_words.data()};
-        DevBuf *dst[3] = {&s.b_probs, &s.b_groups, &s.b_band_probs};
-        size_t at = 0;
-        for (int q = 0; q < 3; q++) {
-            dst[q]->ensure(std::max<size_t>(nb[q], 4));
-            if (!nb[q]) continue;
-            std::memcpy(s.stage + at, src[q], nb[q]);
-            HIPCHK(hipMemcpyAsync(dst[q]->p, s.stage + at, nb[q], hipMemcpyHostToDevice, st));
-            at += (nb[q] + al - 1) / al * al;
-        }
+        s.b_probs.ensure(std::max<size_t>(total, 4));
+        if (nb[0]) std::memcpy(s.stage, pl.probs.data(), nb[0]);
+        if (nb[1]) std::memcpy(s.stage + pc.groups_at, pl.groups.data(), nb[1]);
+        if (nb[2]) std::memcpy(s.stage + pc.bands_at, pl.band_words.data(), nb[2]);
+        if (total) HIPCHK(hipMemcpyAsync(s.b_probs.p, s.stage, total, hipMemcpyHostToDevice, st));
         HIPCHK(hipEventRecord(s.stage_ev, st));
         s.stage_pending = true;
         pc.uploaded = true;
@@ -1698,7 +1699,8 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
     KArgs a;
     std::memset(&a, 0, sizeof(a));  // padding included: the bytes key the graph cache
     a.probs = s.b_probs.as<Prob>();
-    a.groups = s.b_groups.as<Group>();
+    a.groups = reinterpret_cast<const Group *>(s.b_probs.as<char>() + pc.groups_at);
+    const int32_t *band_words = reinterpret_cast<const int32_t *>(s.b_probs.as<char>() + pc.bands_at);
     a.codes_s = codes_s;
     a.codes_t = codes_t;
     a.table = s.b_table.as<float>();
@@ -1750,7 +1752,7 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
     LongArgs la{};
     int long_grid = 0;
     if (plan.n_long > 0) {
-        la.order = s.b_band_probs.as<int32_t>() + n_band;
+        la.order = band_words + n_band;
         la.total_bands = plan.long_bands;
         la.ticket = s.b_queue.as<uint32_t>() + plan.launches.size();
         long_grid = std::max(1, std::min(plan.long_bands, s.cus));
@@ -1772,7 +1774,7 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
             e = launch_long(job.loc, job.dir, job.gap, job.form, job.tr, job.fold_max, a, la, long_grid, st);
         for (size_t q = 0; q < specs.size() && e == hipSuccess; q++) e = launch_solve(specs[q], largs[q], st);
         if (e == hipSuccess && n_band > 0)
-            e = launch_band_combine(job.loc, job.dir, job.tr, s.b_probs.as<Prob>(), s.b_band_probs.as<int32_t>(),
+            e = launch_band_combine(job.loc, job.dir, job.tr, s.b_probs.as<Prob>(), band_words,
                                     n_band, s.b_partials.as<BandPartial>(), scores, seeds, st);
         return e;
     };
@@ -1785,7 +1787,7 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
                                int64_t(reinterpret_cast<intptr_t>(scores)), int64_t(reinterpret_cast<intptr_t>(seeds)),
                                int64_t(job.loc * 100 + job.dir * 10 + job.tr), plan.n_long, plan.long_bands,
                                (plan.xbuf_end - plan.xbuf_begin) * 2 + int64_t(job.fold_max),
-                               int64_t(reinterpret_cast<intptr_t>(s.b_band_probs.p))};
+                               int64_t(reinterpret_cast<intptr_t>(band_words))};
     gkey.append(reinterpret_cast<const char *>(extra), sizeof(extra));
 
     HIPCHK(hipEventRecord(s.ev0, st));
