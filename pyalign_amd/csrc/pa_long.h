@@ -85,7 +85,7 @@ __device__ __forceinline__ constexpr int long_ooff(int w) {
 // costs above zero, so that no candidate is -0 or NaN (x + y is -0 only when
 // both are -0) and max / min keep the strict fold's value.  The strict fold
 // then chooses the first candidate in push order equal to that value, so
-// traceback codes come from equality tests beside the value chain instead
+// traceback codes come from sign tests beside the value chain instead
 // of lengthening it.
 template <int LOC, int DIR, int GAP, int FORM, int TR, bool MX>
 __global__ __launch_bounds__((LONG_WAVES + 1) * WAVE) void pa_long_kernel(KArgs a, LongArgs la) {
@@ -374,14 +374,20 @@ __global__ __launch_bounds__((LONG_WAVES + 1) * WAVE) void pa_long_kernel(KArgs 
                     if constexpr (LOC == LOC_LOCAL) D = opt(D, 0.0f);
                     if constexpr (TR == TR_ONE) {
                         // the first candidate equal to the fold, in push
-                        // order (local: zero, diagonal, vertical, horizontal)
-                        uint32_t src = up == D ? 2u : 3u;
-                        src = dg == D ? 1u : src;
-                        if constexpr (LOC == LOC_LOCAL) src = D == 0.0f ? 0u : src;
-                        bits = src;
+                        // order (local: zero, diagonal, vertical, horizontal),
+                        // as signs (push_sign; the low bit is finished with
+                        // the word, a local cell's at once)
+                        uint32_t b0 = __float_as_uint(lead<DIR>(up, D)), b1 = __float_as_uint(lead<DIR>(dg, D));
+                        if constexpr (LOC == LOC_LOCAL) {
+                            const uint32_t above = __float_as_uint(lead<DIR>(0.0f, D));
+                            b0 = above & (~b1 | b0);
+                            b1 &= above;
+                        }
+                        tacc = push_sign(tacc, __uint_as_float(b0));
+                        tacc = push_sign(tacc, __uint_as_float(b1));
                         if constexpr (GAP == GAP_AFF) {
-                            bits |= better<DIR>(inP + ge_s, inD + go_s) ? 4u : 0u;
-                            bits |= better<DIR>(Ql + ge_t, Dl + go_t) ? 8u : 0u;
+                            tacc = push_sign(tacc, lead<DIR>(inD + go_s, inP + ge_s));
+                            tacc = push_sign(tacc, lead<DIR>(Dl + go_t, Ql + ge_t));
                         }
                     }
                 } else if constexpr (GAP == GAP_LIN) {
@@ -456,8 +462,16 @@ __global__ __launch_bounds__((LONG_WAVES + 1) * WAVE) void pa_long_kernel(KArgs 
                 // never read)
                 if constexpr (TR == TR_ONE) {
                     constexpr int r = t % PK;
-                    tacc = r == 0 ? bits : tacc | (bits << (TB * r));
-                    if constexpr (r == PK - 1) tbq[(t / PK) * WAVE] = tacc;
+                    if constexpr (!MX) tacc = r == 0 ? bits : tacc | (bits << (TB * r));
+                    if constexpr (r == PK - 1) {
+                        uint32_t word = tacc;
+                        if constexpr (MX) {  // the first step's flags to the lowest bits; low bit: diagonal, or not P
+                            constexpr uint32_t LOW = (TB == 4 ? 0x11111111u : 0x55555555u) >> (32 - TB * PK);
+                            word = __builtin_bitreverse32(tacc) >> (32 - TB * PK);
+                            if constexpr (LOC != LOC_LOCAL) word |= ~(word >> 1) & LOW;
+                        }
+                        tbq[(t / PK) * WAVE] = word;
+                    }
                 }
                 Dl = act ? D : Dl;
                 Ql = act ? Q : Ql;
