@@ -477,10 +477,10 @@ class Solver:
         """one(k) -> (form, payload) copies problem k's data for its
         Solution matrices (None: not available)."""
         n = lib().pa_result_count(h)
+        if kind == "score":  # (no lengths to convert)
+            return _Result(h, n, self._index_dtype, (), ()).scores()
         r = _Result(h, n, self._index_dtype, len_s, len_t)
         scores = r.scores()
-        if kind == "score":
-            return scores
         if kind == "alignment":
             if self._opts.count != Count.ONE:
                 return tuple(r.alignment(k, scores[k]) for k in range(n))

@@ -586,7 +586,7 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
     // an eighth of a SIMD's share of the work for the fast kernel, a
     // sixteenth for the general kernel (both measured best)
     // (of a large bag every few problems stand for all)
-    const int64_t stride = std::max<int64_t>(1, n / 1024);
+    const int64_t stride = std::max<int64_t>(1, n / 4096);
     double total = 0.0;
     for (int64_t k = 0; k < n; k += stride) {
         if (ls[k] <= 0 || lt[k] <= 0) continue;
@@ -1899,8 +1899,10 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
     r->goal = o.goal;
     r->index_bits = o.index_bits;
     r->remove_dup = o.remove_dup;
-    r->len_s.assign(in.len_s, in.len_s + n);
-    r->len_t.assign(in.len_t, in.len_t + n);
+    if (job.tr != TR_SCORE) {  // (scores need no lengths)
+        r->len_s.assign(in.len_s, in.len_s + n);
+        r->len_t.assign(in.len_t, in.len_t + n);
+    }
     if (job.tr == TR_ONE) {
         place_results(s, in, st, *r);
         HIPCHK(launch_walk(job.gap, s.b_probs.as<Prob>(), int64_t(plan.probs.size()), s.b_tb.as<uint32_t>(), seeds,
@@ -3103,11 +3105,12 @@ int pa_result_alignments(const pa_result *r, int32_t *s_to_t, int32_t *t_to_s) {
 int pa_result_alignment(const pa_result *r, int64_t k, int32_t *s_to_t, int32_t *t_to_s) {
     return guard([&] {
         if (!r || k < 0 || k >= r->n) fail(PA_EINVAL, "bad problem index");
+        if (r->goal != PA_GOAL_ONE && r->goal != PA_GOAL_ALL) fail(PA_EINVAL, "score-only results carry no alignment");
         const int32_t ls = r->len_s[size_t(k)], lt = r->len_t[size_t(k)];
         if (r->goal == PA_GOAL_ONE) {
             widen(r, r->s_to_t, r->s_at(k), ls, s_to_t);
             widen(r, r->t_to_s, r->t_at(k), lt, t_to_s);
-        } else if (r->goal == PA_GOAL_ALL) {
+        } else {
             const IterState *it = r->iters[size_t(k)].get();
             if (!it || it->cur_path.empty()) fail(PA_EINVAL, "no current alignment");
             std::vector<int32_t> uv;
@@ -3116,8 +3119,6 @@ int pa_result_alignment(const pa_result *r, int64_t k, int32_t *s_to_t, int32_t 
                 uv.push_back(p.second);
             }
             alignment_from_path(uv.data(), int64_t(it->cur_path.size()), ls, lt, s_to_t, t_to_s);
-        } else {
-            fail(PA_EINVAL, "score-only results carry no alignment");
         }
     });
 }
