@@ -1544,6 +1544,25 @@ void build_launches(pa_solver &s, const Job &job, const Input &in, const Plan &p
     }
 }
 
+// Everything that the arguments of a launch sequence are made from (see
+// `enqueue` in run): a captured graph is replayed only where it is the same.
+// `a` and `la` are the arguments of the launches that have no spec (long mode,
+// the band fold, the series check).
+std::string launch_key(const Job &job, const Plan &plan, const std::vector<LaunchSpec> &specs,
+                       const std::vector<KArgs> &largs, const KArgs &a, const LongArgs &la, int long_grid,
+                       const int32_t *band_words, int64_t finite_nx, int64_t finite_ny) {
+    std::string key(reinterpret_cast<const char *>(specs.data()), specs.size() * sizeof(LaunchSpec));
+    key.append(reinterpret_cast<const char *>(largs.data()), largs.size() * sizeof(KArgs));
+    key.append(reinterpret_cast<const char *>(&a), sizeof(a));
+    key.append(reinterpret_cast<const char *>(&la), sizeof(la));
+    const int64_t extra[] = {job.loc, job.dir, job.gap, job.form, job.tr, int64_t(job.fold_max),
+                             int64_t(plan.launches.size()), plan.band_slots, int64_t(plan.band_probs.size()),
+                             plan.n_long, plan.xbuf_begin, plan.xbuf_end, long_grid,
+                             int64_t(reinterpret_cast<intptr_t>(band_words)), finite_nx, finite_ny};
+    key.append(reinterpret_cast<const char *>(extra), sizeof(extra));
+    return key;
+}
+
 void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, float *scores_device,
          pa_tape *tape = nullptr) {
     ensure_device(s);
@@ -1749,7 +1768,8 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
     std::vector<KArgs> largs;
     build_launches(s, job, in, plan, a, s.b_queue.as<uint32_t>(), specs, largs);
     const int n_band = int(plan.band_probs.size());
-    LongArgs la{};
+    LongArgs la;
+    std::memset(&la, 0, sizeof(la));  // (its bytes key the graph cache too)
     int long_grid = 0;
     if (plan.n_long > 0) {
         la.order = band_words + n_band;
@@ -1781,14 +1801,7 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
     // A launch sequence repeated with identical arguments (same shapes, same
     // buffers) is captured once as a hipGraph and replayed; the kernels read
     // the plan and inputs uploaded just before, so a replay sees new data.
-    std::string gkey(reinterpret_cast<const char *>(specs.data()), specs.size() * sizeof(LaunchSpec));
-    gkey.append(reinterpret_cast<const char *>(largs.data()), largs.size() * sizeof(KArgs));
-    const int64_t extra[10] = {int64_t(plan.launches.size()), plan.band_slots, n_band,
-                               int64_t(reinterpret_cast<intptr_t>(scores)), int64_t(reinterpret_cast<intptr_t>(seeds)),
-                               int64_t(job.loc * 100 + job.dir * 10 + job.tr), plan.n_long, plan.long_bands,
-                               (plan.xbuf_end - plan.xbuf_begin) * 2 + int64_t(job.fold_max),
-                               int64_t(reinterpret_cast<intptr_t>(band_words))};
-    gkey.append(reinterpret_cast<const char *>(extra), sizeof(extra));
+    const std::string gkey = launch_key(job, plan, specs, largs, a, la, long_grid, band_words, finite_nx, finite_ny);
 
     HIPCHK(hipEventRecord(s.ev0, st));
     hipError_t le = hipSuccess;

@@ -1,0 +1,80 @@
+// Checks of the library's host code that its C interface does not show
+// (launch keys, plans): run by tests/test_host_checks_cpu.py, no GPU needed.
+// Usage: host_checks CHECK; prints what is wrong, exit status 1 if anything is.
+#include "../pyalign_amd/csrc/pa_api.cpp"
+
+#include <cstdio>
+#include <functional>
+#include <map>
+
+namespace {
+
+int bad = 0;
+
+void expect(bool ok, const std::string &what) {
+    if (ok) return;
+    bad++;
+    std::printf("%s\n", what.c_str());
+}
+
+// One long problem and nothing else: every argument of its launch is in the key.
+void graph_key() {
+    Job job{LOC_GLOBAL, DIR_MAX, GAP_AFF, F_BINARY, TR_ONE, true, false};
+    Plan plan;
+    plan.band_probs = {0};
+    plan.n_long = 1;
+    plan.xbuf_begin = 64;
+    plan.xbuf_end = 128;
+    KArgs a;
+    std::memset(&a, 0, sizeof(a));
+    LongArgs la;
+    std::memset(&la, 0, sizeof(la));
+    int grid = 3;
+    int64_t nx = 5, ny = 6;
+    char memory[16];
+    auto key = [&] { return launch_key(job, plan, {}, {}, a, la, grid, nullptr, nx, ny); };
+    const std::string first = key();
+    expect(key() == first, "the key of the same launches differs");
+    auto changes = [&](const char *what, auto &field, auto value) {
+        const auto old = field;
+        field = value;
+        expect(key() != first, std::string("not in the key: ") + what);
+        field = old;
+    };
+    changes("eq", a.eq, 2.0f);
+    changes("ne", a.ne, -2.0f);
+    changes("go_s", a.go_s, -2.0f);
+    changes("ge_s", a.ge_s, -2.0f);
+    changes("go_t", a.go_t, -2.0f);
+    changes("ge_t", a.ge_t, -2.0f);
+    changes("K1", a.K1, 21);
+    changes("codes_s", a.codes_s, static_cast<const void *>(memory));
+    changes("codes_t", a.codes_t, static_cast<const void *>(memory));
+    changes("table", a.table, reinterpret_cast<const float *>(memory));
+    changes("tb", a.tb, reinterpret_cast<uint32_t *>(memory));
+    changes("rowbuf", a.rowbuf, reinterpret_cast<float2 *>(memory));
+    changes("partials", a.partials, reinterpret_cast<BandPartial *>(memory));
+    changes("border_s", a.border_s, reinterpret_cast<const float *>(memory));
+    changes("order", la.order, reinterpret_cast<const int32_t *>(memory));
+    changes("total_bands", la.total_bands, 7);
+    changes("ticket", la.ticket, reinterpret_cast<uint32_t *>(memory));
+    changes("gap", job.gap, int(GAP_LIN));
+    changes("form", job.form, int(F_TABLE));
+    changes("fold_max", job.fold_max, false);
+    changes("xbuf_begin", plan.xbuf_begin, int64_t(0));
+    changes("grid", grid, 4);
+    changes("finite_nx", nx, int64_t(9));
+    changes("finite_ny", ny, int64_t(9));
+}
+
+}  // namespace
+
+int main(int argc, char **argv) {
+    const std::map<std::string, std::function<void()>> checks = {{"graph_key", graph_key}};
+    if (argc != 2 || !checks.count(argv[1])) {
+        std::printf("usage: host_checks CHECK\n");
+        return 2;
+    }
+    checks.at(argv[1])();
+    return bad ? 1 : 0;
+}
