@@ -1172,12 +1172,23 @@ void fetch_results(pa_solver &s, hipStream_t st, pa_result &r, const float *scor
     HIPCHK(hipMemcpyAsync(r.pin.p, src, bytes, hipMemcpyDeviceToHost, st));
 }
 
-// The table on the device (kept while it repeats).
+bool same_bits(const std::vector<float> &a, const std::vector<float> &b) {
+    return a.size() == b.size() && (a.empty() || std::memcmp(a.data(), b.data(), a.size() * 4) == 0);
+}
+
+// The table on the device, kept while its bits repeat (-0 and +0 fold
+// differently).  An upload that a caller's capture records has not happened
+// yet: it is not counted on.
 void stage_table(pa_solver &s, const Input &in, hipStream_t st) {
-    if (in.table == s.table && s.b_table.p) return;
+    if (s.b_table.p && same_bits(in.table, s.table)) return;
     s.table.clear();
     upload(st, s.b_table, in.table.data(), in.table.size());
-    s.table = in.table;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (s.external_stream && hipStreamIsCapturing(st, &capture) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    if (capture == hipStreamCaptureStatusNone) s.table = in.table;
 }
 
 // Whether a general-gap solve's folds return the strict folds' bits in any
@@ -2660,8 +2671,13 @@ int pa_solver_set_stream(pa_solver *s, void *stream, int32_t external) {
     return guard([&] {
         if (!s) fail(PA_EINVAL, "null solver");
         ensure_device(*s);
+        const hipStream_t before = s->stream;
         s->external_stream = external != 0;
         s->stream = s->external_stream ? static_cast<hipStream_t>(stream) : s->own_stream;
+        if (s->stream != before) {  // copies on the stream left behind may still be on their way
+            s->table.clear();
+            s->off_uploaded = false;
+        }
     });
 }
 
