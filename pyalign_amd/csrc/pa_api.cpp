@@ -1226,14 +1226,14 @@ WsbPlan wsb_plan(const std::vector<Prob> &probs, int cus) {
     WsbPlan plan{};
     plan.n = int64_t(probs.size());
     int64_t widest = 0, problems = 0;
-    int32_t longest = 0;
+    int32_t longest = 0, reach = 0;  // (reach: blocks that a block is pushed to, at most, per direction)
     for (const Prob &pr : probs) {
         const int32_t bs = wsb_blocks(pr.len_s), bt = wsb_blocks(pr.len_t);
         if (!bs || !bt) break;
         problems++;
         widest += std::min(bs, bt);
         longest = std::max(longest, bs + bt);
-        plan.reach = std::max(plan.reach, std::max(bs, bt) - 2);
+        reach = std::max(reach, std::max(bs, bt) - 2);
     }
     // Carried sums cost a load and a store of 256 sums per pair of blocks and
     // pay where an anti-diagonal's blocks are few and have many blocks before
@@ -1247,20 +1247,24 @@ WsbPlan wsb_plan(const std::vector<Prob> &probs, int cus) {
     };
     for (int32_t d = 0;; d++) {
         WsbPlan::Diag g{};
-        int64_t total = 0;
+        int64_t total = 0, sources = 0;  // (sources: groups of four blocks of the anti-diagonal before)
         for (const Prob &pr : probs) {
             const int32_t n = on_diag(pr, d);
             if (!n) break;
             g.problems++;
             g.groups = std::max(g.groups, plan.across ? n : (n + 3) / 4);
-            g.sources = std::max(g.sources, (on_diag(pr, d - 1) + 3) / 4);
+            sources = std::max<int64_t>(sources, (on_diag(pr, d - 1) + 3) / 4);
             total += n;
         }
         if (!g.problems) return plan;
         g.waves = 1;
-        if (plan.carry) g.waves = 2;
-        else  // four waves per SIMD where there is that much to fold
+        if (plan.carry) {
+            g.waves = 2;
+            const int64_t units = sources * 2 * ((reach + WSB_PUSHES - 1) / WSB_PUSHES);
+            g.pushes = int32_t(std::min<int64_t>((units + g.waves - 1) / g.waves, WSB_PUSH_GROUPS));
+        } else {  // four waves per SIMD where there is that much to fold
             while (g.waves < 8 && g.waves < 2 * d && total / 4 * g.waves < 16 * int64_t(cus)) g.waves *= 2;
+        }
         plan.diags.push_back(g);
     }
 }

@@ -291,16 +291,19 @@ hipError_t launch_wsb(int loc, int dir, int form, const KArgs &args, int64_t n, 
 // The problems are sorted by their number of block anti-diagonals, most first;
 // ws / wt have WSB_TILE readable floats past their ends.
 constexpr int WSB_TILE = 16;
+constexpr int WSB_PUSHES = 2;  // distances a wave pushes its four blocks to (carry)
+// Workgroups of one problem that push, at most (two waves each: four per SIMD
+// for a single pair); with more to push they take several turns.
+constexpr int WSB_PUSH_GROUPS = 2048;
 struct WsbPlan {
     int64_t n;     // problems, empty ones included
     bool across;   // a workgroup's four blocks: of four problems (else neighbours of one)
     bool carry;    // every block's values are pushed on once (else later blocks fold all before them)
-    int32_t reach; // carry: blocks that a block is pushed to, at most, per direction
     struct Diag {
         int32_t problems;  // with this anti-diagonal
         int32_t groups;    // workgroups per problem (four problems), at most
         int32_t waves;     // per workgroup, sharing the folds of its four blocks
-        int32_t sources;   // carry: groups of four blocks of the anti-diagonal before, at most, per problem
+        int32_t pushes;    // carry: workgroups per problem that push the anti-diagonal before on
     };
     std::vector<Diag> diags;
 };

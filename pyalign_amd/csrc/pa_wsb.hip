@@ -51,7 +51,6 @@ constexpr int TILE = B * TS;       // floats per block
 constexpr int KS = 2 * B + 1;      // LDS row stride of a solved block (by row and step)
 constexpr int WAVE_LDS = 4 * TILE; // a wave's four blocks
 constexpr int MIN_LDS = 4 * B * KS;
-constexpr int PUSHES = 2;  // distances a wave pushes its four blocks to
 
 // lane r of a row of 16 <- lane r - M; lanes r < M read 0
 template <int M>
@@ -146,38 +145,44 @@ __device__ __forceinline__ float *carried(const KArgs &a, const Prob &pr, int64_
 
 // The blocks of anti-diagonal diag - 1 pushed into the blocks two or more
 // below and to the right of them (those next to them fold them themselves).
-// A wave takes four neighbouring blocks, one direction and PUSHES distances.
+// A unit is four neighbouring blocks, one direction and WSB_PUSHES distances; a
+// wave takes the problem's units from `first` on, `step` apart (a long pair has
+// more than a grid has rows: 16,383 symbols a side 262,000 on one
+// anti-diagonal).
 template <int DIR>
 __device__ __forceinline__ void push_blocks(const KArgs &a, const Prob &pr, const float *__restrict__ ws,
-                                            const float *__restrict__ wt, int diag, int unit, int lane) {
+                                            const float *__restrict__ wt, int diag, int first, int step, int lane) {
     const int ls = pr.len_s, lt = pr.len_t;
     const int nbs = (ls + B - 1) / B, nbt = (lt + B - 1) / B, src = diag - 1;
     const int lo = max(0, src - nbt + 1), hi = min(src, nbs - 1);
     if (lo > hi) return;
     const int groups = (hi - lo + 4) / 4;
-    const int g = unit % groups, down = unit / groups % 2, x0 = 2 + unit / groups / 2 * PUSHES;
+    // distances 2 .. the farthest of the anti-diagonal's blocks, in either direction
+    const int farthest = max(nbs - 1 - lo, nbt - 1 - (src - hi));
+    const int units = farthest < 2 ? 0 : groups * 2 * ((farthest - 1 + WSB_PUSHES - 1) / WSB_PUSHES);
     const int q = lane >> 4, l = lane & (B - 1);
-    const int bi = lo + 4 * g + q, bj = src - bi;
-    if (bi > hi) return;
-    const int reach = down ? nbs - 1 - bi : nbt - 1 - bj;  // blocks below / to the right
-    if (x0 > reach) return;
     const int64_t cells = int64_t(ls) * lt;
     const float *D = a.dvals + pr.dv_off, *DT = D + cells;
-    const bool first = (down ? bi : bj) == 0;  // the target's first candidates
-    float v[B];
-    if (down) load_block(D + int64_t(B) * bi * lt + min(B * bj + l, lt - 1), lt, v);
-    else load_block(DT + int64_t(B) * bj * ls + min(B * bi + l, ls - 1), ls, v);
-    for (int x = x0; x < x0 + PUSHES; ++x) {
-        if (x > reach) return;
-        float *acc_at = carried(a, pr, down ? int64_t(bi + x) * nbt + bj : int64_t(bi) * nbt + bj + x) +
-                        (down ? 0 : B * B) + l;
-        float acc[B];
+    for (int unit = first; unit < units; unit += step) {
+        const int g = unit % groups, down = unit / groups % 2, x0 = 2 + unit / groups / 2 * WSB_PUSHES;
+        const int bi = lo + 4 * g + q, bj = src - bi;
+        const int reach = bi > hi ? 0 : (down ? nbs - 1 - bi : nbt - 1 - bj);  // blocks below / to the right
+        if (x0 > reach) continue;
+        const bool start = (down ? bi : bj) == 0;  // the target's first candidates
+        float v[B];
+        if (down) load_block(D + int64_t(B) * bi * lt + min(B * bj + l, lt - 1), lt, v);
+        else load_block(DT + int64_t(B) * bj * ls + min(B * bi + l, ls - 1), ls, v);
+        for (int x = x0; x < x0 + WSB_PUSHES && x <= reach; ++x) {
+            float *acc_at = carried(a, pr, down ? int64_t(bi + x) * nbt + bj : int64_t(bi) * nbt + bj + x) +
+                            (down ? 0 : B * B) + l;
+            float acc[B];
 #pragma unroll
-        for (int r = 0; r < B; ++r) acc[r] = first ? worst<DIR>() : acc_at[r * B];
-        if (down) fold_block<DIR>(v, ws + B * x, acc);
-        else fold_block<DIR>(v, wt + B * x, acc);
+            for (int r = 0; r < B; ++r) acc[r] = start ? worst<DIR>() : acc_at[r * B];
+            if (down) fold_block<DIR>(v, ws + B * x, acc);
+            else fold_block<DIR>(v, wt + B * x, acc);
 #pragma unroll
-        for (int r = 0; r < B; ++r) acc_at[r * B] = acc[r];
+            for (int r = 0; r < B; ++r) acc_at[r * B] = acc[r];
+        }
     }
 }
 
@@ -198,7 +203,8 @@ __global__ __launch_bounds__(512) void pa_wsb_block_kernel(KArgs a, const float 
     const int waves = int(blockDim.x) / WAVE;
     const int lane = int(threadIdx.x) & (WAVE - 1);
     if (int(blockIdx.y) >= groups) {
-        push_blocks<DIR>(a, a.probs[blockIdx.x], ws, wt, diag, (int(blockIdx.y) - groups) * waves + wave, lane);
+        push_blocks<DIR>(a, a.probs[blockIdx.x], ws, wt, diag, (int(blockIdx.y) - groups) * waves + wave,
+                         (int(gridDim.y) - groups) * waves, lane);
         return;
     }
     const int q = lane >> 4, l = lane & (B - 1);
@@ -530,11 +536,8 @@ hipError_t launch_blocks(const KArgs &a, const WsbPlan &plan, const float *ws, c
     for (size_t d = 0; d < plan.diags.size(); ++d) {
         const WsbPlan::Diag &g = plan.diags[d];
         const int x = plan.across ? (g.problems + 3) / 4 : g.problems;
-        // each push workgroup holds `waves` units of (four blocks, direction, PUSHES distances)
-        const int units = plan.carry && d > 0 ? g.sources * 2 * ((plan.reach + PUSHES - 1) / PUSHES) : 0;
         hipLaunchKernelGGL((pa_wsb_block_kernel<LOC, DIR, FORM>),
-                           dim3(unsigned(x), unsigned(g.groups + (units + g.waves - 1) / g.waves)),
-                           dim3(unsigned(g.waves * WAVE)),
+                           dim3(unsigned(x), unsigned(g.groups + g.pushes)), dim3(unsigned(g.waves * WAVE)),
                            std::max(size_t(g.waves) * WAVE_LDS, size_t(MIN_LDS)) * 4, st, a, ws, wt, int(d),
                            int(g.problems), int(g.groups), int(plan.across), int(plan.carry));
         const hipError_t e = hipGetLastError();

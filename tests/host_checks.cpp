@@ -67,10 +67,36 @@ void graph_key() {
     changes("finite_ny", ny, int64_t(9));
 }
 
+// General gap costs: every launch of long pairs fits a grid (its y extent is
+// 65,535 at most) and has workgroups for what it pushes on.
+void wsb_extents() {
+    const std::vector<std::vector<std::pair<int, int>>> bags = {
+        {{11600, 11600}}, {{16383, 16383}}, {{32000, 32000}}, {{400, 300000}}, {{1, 3000000}}, {{3000000, 1}},
+        {{700, 700}, {30, 40}, {5, 2000000}}};
+    for (const auto &bag : bags) {
+        std::vector<Prob> probs;
+        for (const auto &shape : bag) {
+            Prob pr{};
+            pr.len_s = shape.first;
+            pr.len_t = shape.second;
+            probs.push_back(pr);
+        }
+        std::stable_sort(probs.begin(), probs.end(), [](const Prob &x, const Prob &y) {
+            return wsb_blocks(x.len_s) + wsb_blocks(x.len_t) > wsb_blocks(y.len_s) + wsb_blocks(y.len_t);
+        });
+        const WsbPlan plan = wsb_plan(probs, 256);
+        const std::string name = std::to_string(bag[0].first) + " x " + std::to_string(bag[0].second);
+        expect(plan.carry, name + ": no carried sums");
+        int64_t most = 0;
+        for (const WsbPlan::Diag &g : plan.diags) most = std::max(most, int64_t(g.groups) + g.pushes);
+        expect(most > 1 && most <= 65535, name + ": " + std::to_string(most) + " workgroups in y");
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"graph_key", graph_key}};
+    const std::map<std::string, std::function<void()>> checks = {{"graph_key", graph_key}, {"wsb_extents", wsb_extents}};
     if (argc != 2 || !checks.count(argv[1])) {
         std::printf("usage: host_checks CHECK\n");
         return 2;
