@@ -1016,21 +1016,25 @@ struct Input {
     bool table_g = false;
 };
 
-// Whether max / min folds (and traceback codes from equality tests) keep the
-// strict folds' bits in alignments over a table, binary symbols or a dense
-// matrix:
-// similarities finite (or the pad's worst value) and never -0, and, for
-// maximising global problems, gap costs above zero (borders below -0), so that
-// no candidate is -0 or NaN.
+// Whether max / min folds (and traceback codes from the signs of differences)
+// keep the strict folds' bits in alignments over a table, binary symbols or a
+// dense matrix, that is, no candidate can be -0 or NaN and no value infinite:
+// * gap costs at most 1e30 (borders and gaps stay finite, and a cell is never
+//   worse than a gap from its neighbour) and similarities no better than 1e30
+//   (sums stay finite); worse ones may be anything, the direction's worst
+//   value and the largest number of the other sign included;
+// * no similarity -0, and, for maximising global problems, gap costs above
+//   zero (borders below -0).
 bool folds_max(const pa_solver &s, const Input &in, const Job &job) {
     if (job.gap != GAP_LIN && job.gap != GAP_AFF) return false;
-    auto exact = [](float x) { return std::isfinite(x) && !(x == 0.0f && std::signbit(x)); };
+    for (float cost : {s.go_s, s.ge_s, s.go_t, s.ge_t})
+        if (!(std::fabs(cost) <= 1e30f)) return false;
     if (job.loc == LOC_GLOBAL && job.dir == DIR_MAX && !(s.go_s < 0.0f && s.go_t < 0.0f)) return false;
-    if (job.form == F_BINARY) return exact(in.eq) && exact(in.ne);
+    const float sgn = job.dir == DIR_MAX ? 1.0f : -1.0f;
+    auto exact = [&](float x) { return sgn * x <= 1e30f && !(x == 0.0f && std::signbit(x)); };
+    if (job.form == F_BINARY) return std::isfinite(in.eq) && std::isfinite(in.ne) && exact(in.eq) && exact(in.ne);
     if (job.form == F_DENSE) return true;  // (the kernel looks at the values and falls back)
-    if (job.form != F_TABLE) return false;
-    const float w = worst(s.opt.dir);
-    return std::all_of(in.table.begin(), in.table.end(), [&](float x) { return exact(x) || x == w; });
+    return job.form == F_TABLE && std::all_of(in.table.begin(), in.table.end(), exact);
 }
 
 // Whether the score kernel serves a job.  The local maximum over a table needs

@@ -44,8 +44,9 @@ __device__ __forceinline__ float opt(float a, float b) {
 }
 
 // Traceback flags without lane masks: the sign of lead(a, b) says that b is
-// strictly better than a (their difference is exact in sign; equal values,
-// infinities too, give +0 or a positive NaN), and push_sign shifts it into a
+// strictly better than a (their difference is exact in sign, and +0 for equal
+// values; two infinities of one sign give a NaN of either sign, so the caller
+// keeps them out), and push_sign shifts it into a
 // word with one v_alignbit_b32.  A compare, its 64-bit mask in scalar
 // registers and a select of a constant cost as many instructions and the wait
 // states between mask and select (38 s_nop in an 8-cell Gotoh step; 2,048 local

@@ -93,10 +93,47 @@ void wsb_extents() {
     }
 }
 
+// Which gap costs and similarities max / min folds are chosen for.
+void fold_rule() {
+    const float inf = std::numeric_limits<float>::infinity(), huge = std::numeric_limits<float>::max(),
+                nan = std::numeric_limits<float>::quiet_NaN();
+    for (int dir : {DIR_MAX, DIR_MIN}) {
+        const float sgn = dir == DIR_MAX ? 1.0f : -1.0f;
+        pa_solver s;
+        s.opt.dir = dir == DIR_MAX ? PA_MAXIMIZE : PA_MINIMIZE;
+        auto folds = [&](float open, float extend, std::vector<float> values, int form = F_TABLE, int loc = LOC_SEMI) {
+            s.go_s = s.go_t = -sgn * open;
+            s.ge_s = s.ge_t = -sgn * extend;
+            Input in{};
+            for (float &x : values) x = x == 0.0f ? x : sgn * x;
+            in.table = values;
+            in.eq = values[0];
+            in.ne = values[1];
+            return folds_max(s, in, Job{loc, dir, GAP_AFF, form, TR_ONE, false, false});
+        };
+        for (int form : {F_TABLE, F_BINARY}) {
+            const std::string name = (form == F_TABLE ? "table, " : "binary, ") + std::to_string(dir) + ": ";
+            expect(folds(3, 1, {2, -1}, form), name + "usual values refused");
+            expect(folds(0, 0, {2, 0}, form), name + "free gaps refused");
+            expect(folds(3, 1, {2, -huge}, form), name + "the lowest value refused");
+            expect(!folds(inf, 1, {2, -1}, form), name + "an infinite open cost taken");
+            expect(!folds(3, inf, {2, -1}, form), name + "an infinite extension taken");
+            expect(!folds(nan, 1, {2, -1}, form), name + "a NaN cost taken");
+            expect(!folds(3, 1, {huge, -1}, form), name + "a sum that overflows taken");
+            expect(!folds(3, 1, {2, nan}, form), name + "NaN taken");
+            expect(!folds(3, 1, {2, -0.0f}, form), name + "-0 taken");
+            expect(!folds(3, 1, {inf, -1}, form), name + "an infinite match taken");
+        }
+        expect(folds(3, 1, {2, -inf}), "the worst value in a table refused");
+        expect(!folds(inf, 1, {2, -1}, F_DENSE), "dense with an infinite cost taken");
+        expect(folds(0, 1, {2, -1}, F_TABLE, LOC_GLOBAL) == (dir == DIR_MIN), "global, free opening");
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"graph_key", graph_key}, {"wsb_extents", wsb_extents}};
+    const std::map<std::string, std::function<void()>> checks = {{"graph_key", graph_key}, {"wsb_extents", wsb_extents}, {"fold_rule", fold_rule}};
     if (argc != 2 || !checks.count(argv[1])) {
         std::printf("usage: host_checks CHECK\n");
         return 2;
