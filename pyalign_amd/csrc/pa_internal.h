@@ -169,11 +169,14 @@ struct KArgs {
     const float *safe;
     // SINK_WORDS writable words: where a lane with nothing to store stores
     uint32_t *sink;
-    // series form (DTW): a word that holds 1 when every series value is
-    // finite, so that the cells' costs and values are never NaN or -0 and
-    // min / max folds return the strict folds' bits (null: strict folds)
+    // series form (DTW): a word that holds 1 when no series value exceeds
+    // SERIES_MOST, so that the cells' costs and values are finite and never -0
+    // and min / max folds return the strict folds' bits (null: strict folds)
     const uint32_t *finite;
 };
+// squared differences of four dimensions, summed along any path, stay below
+// float32's largest value: 4 (2e13)^2 2^31 = 3.4e36
+constexpr float SERIES_MOST = 1e13f;
 constexpr int SAFE_FLOATS = 16;
 constexpr int SINK_WORDS = 16;
 
@@ -262,7 +265,8 @@ struct StripWalk {
 hipError_t launch_backward_strips(int gap, int form, int dim, const BwArgs &args, StripWalk *state,
                                   const int32_t *strip_of, hipStream_t stream);
 hipError_t launch_fill_u32(uint32_t *p, int64_t n, uint32_t value, hipStream_t stream);
-// *flag = 1 when the nx floats at x and the ny floats at y are all finite, else 0
+// *flag = 1 when the nx floats at x and the ny floats at y are all at most
+// SERIES_MOST in magnitude, else 0
 hipError_t launch_all_finite(const float *x, int64_t nx, const float *y, int64_t ny, uint32_t *flag,
                              hipStream_t stream);
 // Raw symbols (width 1 or 4 bytes) to codes: uint8 or uint16 (out_width 1,
