@@ -109,8 +109,13 @@ __device__ __forceinline__ void band_wait(const KArgs &a, int idx, uint32_t need
 
 extern __shared__ float pa_dyn_lds[];  // the launch's dynamic LDS (table or staging windows)
 
-// Returns whether the group's results stand: false where a dense similarity
-// met by max / min folds is infinite, NaN or -0, which only strict folds take.
+// Returns whether the group's results stand: false where max / min folds met a
+// dense similarity that only strict folds take.  Those are NaN and values
+// better than 1e30 (sums could become infinite); masks of the worst value, or
+// of the lowest number, are none.  Nor is -0, except in one cell: a sum is -0
+// only where both its terms are, so without a -0 in the borders no value
+// becomes one, and of the borders only D(-1, -1) of maximising global problems
+// is -0 (gap costs above zero), which S(0, 0) alone is added to.
 template <int LOC, int DIR, int GAP, int FORM, int TR, int R, int SD, int VAR, bool BAND = false>
 __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, const float *__restrict__ tab,
                                             int lane) {
@@ -119,6 +124,7 @@ __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, cons
     constexpr bool TABLE = FORM == F_TABLE || FORM == F_TABLE_G;  // tab: LDS or global memory
     constexpr bool STAGED = FORM == F_DROWS;
     static_assert(!STAGED || R == DROWS_WIN, "staged dense rows need R == 8");
+    constexpr bool WATCH = VAR == VAR_MAX && DENSE;
     constexpr int BITS = TR == TR_ALL ? 8 : (TR == TR_ONE ? (GAP == GAP_AFF ? 4 : 2) : 0);
     constexpr int WPC = TR == TR_SCORE ? 1 : (BITS * R + 31) / 32;
     constexpr int SDD = SD > 0 ? SD : 1;
@@ -356,6 +362,9 @@ __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, cons
 #pragma unroll
             for (int q = 0; q < 4; ++q) wload(1, q, stg[q]);
         }
+        if constexpr (WATCH && LOC == LOC_GLOBAL && DIR == DIR_MAX) {
+            if (st == 0) odd_value |= act && l == 0 && __float_as_uint(STAGED ? *lw : cA.S[0]) == 0x80000000u;
+        }
 
         // one step: column j = s - l of this lane's R rows; the left column
         // D(i, j-1) is read from Din and this column written to Dout (two
@@ -450,8 +459,8 @@ __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, cons
                         if constexpr (PADW) S = rv[r] ? S : W;
                     } else if constexpr (DENSE) {
                         S = PADW ? (rv[r] ? Scol[r] : W) : Scol[r];
-                        // NaN, infinities, -0 (in padded rows as well: their loads read valid memory)
-                        if constexpr (VAR == VAR_MAX) odd_value |= __builtin_amdgcn_classf(Scol[r], 0x227);
+                        // (padded rows read row 0, lanes without a problem the worst value)
+                        if constexpr (WATCH) odd_value |= !(DIR == DIR_MAX ? Scol[r] <= 1e30f : Scol[r] >= -1e30f);
                     } else {
                         // squared Euclidean cost, dimensions summed in order
                         float c = 0.0f;
@@ -662,11 +671,12 @@ __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, cons
         // kernels of their own, VAR_MAX: a kernel holds the registers of its
         // largest loop, 256 and a wave per SIMD where these shared one)
         using Gen = integral_constant<bool, false>;
+        auto watched = [&] { return WATCH && __any(odd_value); };  // (the sweep is for nothing)
         auto sweep = [&](auto kv) {
             int s = 0;
             if constexpr (STAGED) {
                 // eight steps a round: the phase s % 8 is a compile-time constant
-                for (; s < steps; s += 8) {
+                for (; s < steps && !watched(); s += 8) {
                     step(Gen{}, integral_constant<int, 0>{}, kv, s, DlA, DlB, cA);
                     if (s + 1 < steps) step(Gen{}, integral_constant<int, 1>{}, kv, s + 1, DlB, DlA, cB);
                     if (s + 2 < steps) step(Gen{}, integral_constant<int, 2>{}, kv, s + 2, DlA, DlB, cA);
@@ -690,14 +700,14 @@ __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, cons
                             step(Gen{}, integral_constant<int, 0>{}, kv, s, DlA, DlB, cA);
                             step(Gen{}, integral_constant<int, 0>{}, kv, s + 1, DlB, DlA, cB);
                         }
-                        for (int k = (sb - sa) >> 1; k > 0; --k, s += 2) {  // a uniform trip count
+                        for (int k = (sb - sa) >> 1; k > 0 && !watched(); --k, s += 2) {  // a uniform trip count
                             step(integral_constant<bool, true>{}, integral_constant<int, 0>{}, kv, s, DlA, DlB, cA);
                             step(integral_constant<bool, true>{}, integral_constant<int, 0>{}, kv, s + 1, DlB, DlA,
                                  cB);
                         }
                     }
                 }
-                for (; s + 1 < steps; s += 2) {
+                for (; s + 1 < steps && !watched(); s += 2) {
                     step(Gen{}, integral_constant<int, 0>{}, kv, s, DlA, DlB, cA);
                     step(Gen{}, integral_constant<int, 0>{}, kv, s + 1, DlB, DlA, cB);
                 }
@@ -731,6 +741,7 @@ __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, cons
         } else {
             sweep(integral_constant<int, 0>{});
         }
+        if (watched()) return false;
         if constexpr (LOC == LOC_GLOBAL) {
             // D(ls-1, lt-1): column lt-1 was this lane's step lt-1+l, which
             // wrote DlB when even and DlA when odd; later steps write nothing
@@ -815,7 +826,7 @@ __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, cons
             }
         }
     }
-    return !(VAR == VAR_MAX && DENSE) || !__any(odd_value);
+    return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -1208,8 +1219,8 @@ __global__ __launch_bounds__(256) void pa_solve_kernel(KArgs a) {
                 continue;
             }
         }
-        // dense similarities are not known beforehand: max / min folds that
-        // watch for values they cannot take, and strict folds after those
+        // dense similarities are not known beforehand: max / min folds stop at
+        // a value that they cannot take, and strict folds start over
         if (!solve_group<LOC, DIR, GAP, FORM, TR, R, SD, VAR>(a, g, tab, lane)) {
             if constexpr (DENSE_MAX) solve_group<LOC, DIR, GAP, FORM, TR, R, SD, VAR_PLAIN>(a, g, tab, lane);
         }
