@@ -1176,6 +1176,16 @@ void fetch_results(pa_solver &s, hipStream_t st, pa_result &r, const float *scor
     HIPCHK(hipMemcpyAsync(r.pin.p, src, bytes, hipMemcpyDeviceToHost, st));
 }
 
+// whether a caller's capture records the stream's work (or may: the query fails)
+bool recorded(const pa_solver &s, hipStream_t st) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (s.external_stream && hipStreamIsCapturing(st, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return status != hipStreamCaptureStatusNone;
+}
+
 bool same_bits(const std::vector<float> &a, const std::vector<float> &b) {
     return a.size() == b.size() && (a.empty() || std::memcmp(a.data(), b.data(), a.size() * 4) == 0);
 }
@@ -1187,20 +1197,19 @@ void stage_table(pa_solver &s, const Input &in, hipStream_t st) {
     if (s.b_table.p && same_bits(in.table, s.table)) return;
     s.table.clear();
     upload(st, s.b_table, in.table.data(), in.table.size());
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (s.external_stream && hipStreamIsCapturing(st, &capture) != hipSuccess) {
-        (void)hipGetLastError();
-        return;
-    }
-    if (capture == hipStreamCaptureStatusNone) s.table = in.table;
+    if (!recorded(s, st)) s.table = in.table;
 }
 
 // Whether a general-gap solve's folds return the strict folds' bits in any
 // order: similarities and costs finite (sums cannot overflow) or, for
 // similarities, the worst value, and no candidate -0 (a sum is -0 only where
 // both terms are: no similarity is, and not both a border cell and a cost).
-// Device-resident dense similarities are not read here: false.
-bool wsb_any_order(const pa_solver &s, const Input &in, const Job &job) {
+// Dense similarities given on the device are not read here: false.  `dense` is
+// the device copy of those given on the host: many of them are looked at there,
+// where it takes no time (41 million values: 46 ms on one host thread, which is
+// more than the blocks save; few, or under a caller's capture, which cannot
+// wait for the answer: on the host).
+bool wsb_any_order(pa_solver &s, const Input &in, const Job &job, const float *dense, hipStream_t st) {
     auto finite = [](float x) { return std::fabs(x) <= 1e30f; };
     auto neg0 = [](float x) { return x == 0.0f && std::signbit(x); };
     bool cost0 = false, border0 = false;
@@ -1218,8 +1227,17 @@ bool wsb_any_order(const pa_solver &s, const Input &in, const Job &job) {
     if (job.form == F_BINARY) return finite(in.eq) && finite(in.ne) && !neg0(in.eq) && !neg0(in.ne);
     const float w = worst(s.opt.dir);
     auto good = [&](float x) { return (finite(x) && !neg0(x)) || x == w; };
-    if (job.form == F_DENSE)
-        return !in.on_device && std::all_of(in.dense, in.dense + in.dense_elems, good);
+    if (job.form == F_DENSE) {
+        if (in.on_device) return false;
+        if (in.dense_elems < (1 << 15) || recorded(s, st))
+            return std::all_of(in.dense, in.dense + in.dense_elems, good);
+        s.b_finite.ensure(4);
+        uint32_t flag = 0;
+        HIPCHK(launch_any_order(dense, in.dense_elems, w, s.b_finite.as<uint32_t>(), st));
+        HIPCHK(hipMemcpyAsync(&flag, s.b_finite.p, 4, hipMemcpyDeviceToHost, st));
+        HIPCHK(hipStreamSynchronize(st));
+        return flag != 0;
+    }
     return std::all_of(in.table.begin(), in.table.end(), good);
 }
 
@@ -1284,7 +1302,10 @@ void run_wsb(pa_solver &s, const Input &in, const Job &job, std::unique_ptr<pa_r
     const int64_t n = in.n;
     if (!s.gen_ready) fail(PA_EINVAL, "general gap costs were not given to the solver");
     hipStream_t st = s.stream;
-    const bool blocks = job.tr != TR_ALL && !in.matrices && wsb_any_order(s, in, job);
+    const void *codes_s = nullptr, *codes_t = nullptr;
+    const float *dense = nullptr;
+    stage_payload(s, in, st, codes_s, codes_t, dense);
+    const bool blocks = job.tr != TR_ALL && !in.matrices && wsb_any_order(s, in, job, dense, st);
     std::vector<Prob> probs(static_cast<size_t>(n));
     int64_t words = 0;
     double cells = 0;
@@ -1334,9 +1355,6 @@ void run_wsb(pa_solver &s, const Input &in, const Job &job, std::unique_ptr<pa_r
     s.b_wt.ensure((s.wt_sgn.size() + WSB_TILE) * 4);
     upload(st, s.b_ws, s.ws_sgn.data(), s.ws_sgn.size());
     upload(st, s.b_wt, s.wt_sgn.data(), s.wt_sgn.size());
-    const void *codes_s = nullptr, *codes_t = nullptr;
-    const float *dense = nullptr;
-    stage_payload(s, in, st, codes_s, codes_t, dense);
     if (job.form == F_TABLE || job.form == F_TABLE_G) stage_table(s, in, st);
     s.b_dvals.ensure(size_t(std::max<int64_t>(words, 1)) * 4);
     float *scores = scores_device;

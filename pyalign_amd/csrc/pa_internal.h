@@ -269,6 +269,9 @@ hipError_t launch_fill_u32(uint32_t *p, int64_t n, uint32_t value, hipStream_t s
 // SERIES_MOST in magnitude, else 0
 hipError_t launch_all_finite(const float *x, int64_t nx, const float *y, int64_t ny, uint32_t *flag,
                              hipStream_t stream);
+// *flag = 1 when each of the n floats at x is `w` or at most 1e30 in magnitude
+// and not -0, else 0
+hipError_t launch_any_order(const float *x, int64_t n, float w, uint32_t *flag, hipStream_t stream);
 // Raw symbols (width 1 or 4 bytes) to codes: uint8 or uint16 (out_width 1,
 // 2) through lut, or uint32 values (out_width 4) when lut is null; *bad gets
 // the smallest position without a code.

@@ -1578,23 +1578,45 @@ hipError_t launch_fill_u32(uint32_t *p, int64_t n, uint32_t value, hipStream_t s
 
 hipError_t launch_zero_u32(uint32_t *p, int64_t n, hipStream_t st) { return launch_fill_u32(p, n, 0u, st); }
 
-// flag (set to 1 beforehand) cleared when a value is NaN or its magnitude above SERIES_MOST
-__global__ __launch_bounds__(256) void pa_all_finite_kernel(const float *x, int64_t nx, const float *y, int64_t ny,
-                                                            uint32_t *flag) {
+// flag (set to 1 beforehand) cleared when a value is not good; bound by memory
+template <class Good>
+__device__ __forceinline__ void check_all(const float *x, int64_t nx, const float *y, int64_t ny, uint32_t *flag,
+                                          Good &&good) {
     bool bad = false;
     const int64_t stride = int64_t(gridDim.x) * blockDim.x;
     for (int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; k < nx + ny; k += stride)
-        bad = bad || !(fabsf(k < nx ? x[k] : y[k - nx]) <= SERIES_MOST);
+        bad = bad || !good(k < nx ? x[k] : y[k - nx]);
     if (__any(bad) && (threadIdx.x & (WAVE - 1)) == 0)
         __hip_atomic_store(flag, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ __launch_bounds__(256) void pa_all_finite_kernel(const float *x, int64_t nx, const float *y, int64_t ny,
+                                                            uint32_t *flag) {
+    check_all(x, nx, y, ny, flag, [](float v) { return fabsf(v) <= SERIES_MOST; });
+}
+
+__global__ __launch_bounds__(256) void pa_any_order_kernel(const float *x, int64_t n, float w, uint32_t *flag) {
+    check_all(x, n, nullptr, 0, flag, [w](float v) {
+        return (fabsf(v) <= 1e30f && __float_as_uint(v) != 0x80000000u) || v == w;
+    });
+}
+
+static dim3 check_grid(int64_t n) {
+    return dim3(unsigned(std::min<int64_t>((n + 255) / 256, int64_t(device_cus()) * 8)));
 }
 
 hipError_t launch_all_finite(const float *x, int64_t nx, const float *y, int64_t ny, uint32_t *flag,
                              hipStream_t st) {
     hipError_t e = launch_fill_u32(flag, 1, 1u, st);
     if (e != hipSuccess || nx + ny == 0) return e;
-    const int64_t blocks = std::min<int64_t>((nx + ny + 255) / 256, int64_t(device_cus()) * 8);
-    hipLaunchKernelGGL(pa_all_finite_kernel, dim3(unsigned(blocks)), dim3(256), 0, st, x, nx, y, ny, flag);
+    hipLaunchKernelGGL(pa_all_finite_kernel, check_grid(nx + ny), dim3(256), 0, st, x, nx, y, ny, flag);
+    return hipGetLastError();
+}
+
+hipError_t launch_any_order(const float *x, int64_t n, float w, uint32_t *flag, hipStream_t st) {
+    hipError_t e = launch_fill_u32(flag, 1, 1u, st);
+    if (e != hipSuccess || n == 0) return e;
+    hipLaunchKernelGGL(pa_any_order_kernel, check_grid(n), dim3(256), 0, st, x, n, w, flag);
     return hipGetLastError();
 }
 
