@@ -1566,6 +1566,11 @@ void build_launches(pa_solver &s, const Job &job, const Input &in, const Plan &p
             waves_per_cu = std::max(1, occupancy_waves(spec, in.dim));
             s.occ_cache.push_back({okey, waves_per_cu});
         }
+        // Band-mode strips wait for the strips above them: a third wave per SIMD
+        // (DTW's traceback build has the registers for it) mostly polls and
+        // slows the other two.  1,039 DTW pairs of 500 to 2,000, nearly all in
+        // strips: two waves 5.0 ms, three 5.8 ms.
+        if (!fastmax && int64_t(plan.band_probs.size()) > plan.n_long) waves_per_cu = std::min(waves_per_cu, 8);
         // the fast kernel's large workgroups only where the groups fill every
         // CU with them; fewer groups spread over more, smaller workgroups
         spec.block = fastmax && R == 0 && int64_t(g1 - g0) >= int64_t(s.cus) * (FAST_BLOCK / WAVE) ? FAST_BLOCK : 256;
