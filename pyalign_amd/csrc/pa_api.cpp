@@ -190,6 +190,7 @@ struct Plan {
     int32_t long_bands = 0;            // their bands (workgroup tickets)
     std::vector<int32_t> band_words;   // device copy: band_probs, then (problem, band) of every ticket
     int64_t xbuf_begin = 0, xbuf_end = 0;  // float2 range of the row buffer holding their tagged hand-offs
+    bool ckpt = false;                     // some problems keep no traceback (a checkpointed forward)
 };
 
 // The last call's schedule, reused (with its device copy) while the next
@@ -777,6 +778,7 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
         items.swap(sorted);
     }
     Plan plan;
+    plan.ckpt = ckpt != nullptr;
     plan.probs.reserve(static_cast<size_t>(n));
     struct GroupR {
         Group g;
@@ -1546,6 +1548,7 @@ void build_launches(pa_solver &s, const Job &job, const Input &in, const Plan &p
         spec.fastmax = fastmax;
         spec.lds_bytes = job.form == F_TABLE ? size_t(in.K1) * in.K1 * 4 : 0;
         spec.var = job.tr == TR_SCORE ? VAR_PLAIN : a.dvals ? VAR_VALUES : job.fold_max ? VAR_MAX : VAR_PLAIN;
+        if (job.gap == GAP_DTW && plan.ckpt) spec.var = VAR_CKPT;
         if (drows && R == DROWS_WIN) {
             spec.form = F_DROWS;
             spec.lds_bytes = DROWS_LDS;
@@ -2786,6 +2789,7 @@ void backward_checkpointed(pa_tape &t, const BwArgs &base, int form, hipStream_t
     spec.form = t.form;
     spec.tr = TR_ONE;
     spec.R = BAND_R;
+    spec.var = t.gap == GAP_DTW ? VAR_CKPT : VAR_PLAIN;
     const int waves_per_cu = std::max(1, occupancy_waves(spec, t.dim));
     t.s_progress.ensure(size_t(std::max<int64_t>(t.band_slots, 1)) * 4);
     t.s_partials.ensure(size_t(std::max<int64_t>(t.band_slots, 1)) * sizeof(BandPartial));

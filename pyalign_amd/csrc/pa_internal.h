@@ -29,8 +29,13 @@ constexpr size_t DROWS_LDS = size_t(256) * DROWS_LANE_FLOATS * 4;
 enum { TR_SCORE = 0, TR_ONE = 1, TR_ALL = 2 };
 // Builds of the general kernel that keeps a traceback: the usual one, one that
 // also stores cell values (KArgs::dvals), and alignments over a table, binary
-// symbols or a dense matrix with max / min folds.
-enum { VAR_PLAIN = 0, VAR_VALUES = 1, VAR_MAX = 2 };
+// symbols or a dense matrix with max / min folds.  DTW launches of or for a
+// checkpointed forward have one for two waves per SIMD: their longest pairs
+// bound them, which a third wave and the fewer registers it leaves slow down
+// (3,000 training pairs of 1,000 to 4,000: 23.1 -> 20.5 ms a step; 8,192 of 128
+// to 4,096 27.5 -> 26.8), where bags of like pairs gain by it (5,000 of 900 to
+// 1,000: 2.8 -> 2.5 ms).
+enum { VAR_PLAIN = 0, VAR_VALUES = 1, VAR_MAX = 2, VAR_CKPT = 3 };
 
 constexpr int WAVE = 64;
 constexpr int MAX_LDS_TABLE = 129;  // K + 1 pad symbol

@@ -666,7 +666,7 @@ __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, cons
         // carries no per-cell test: 0 codes stored, 1 codes and cell values
         // (a.dvals; kernels of their own, VAR_VALUES), 2 neither (the groups of
         // a checkpointed forward keep strip rows only; their folds keep their
-        // order, their codes go); 3 and 4 as 0 and 2 with min / max folds (DTW
+        // order, their codes go; DTW: VAR_CKPT); 3 and 4 as 0 and 2 with min / max folds (DTW
         // over finite series; alignment over tables and binary symbols in
         // kernels of their own, VAR_MAX: a kernel holds the registers of its
         // largest loop, 256 and a wave per SIMD where these shared one)
@@ -722,7 +722,8 @@ __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, cons
         } else if constexpr (VAR == VAR_MAX) {
             sweep(integral_constant<int, 3>{});
         } else if constexpr (TR == TR_ONE) {
-            const bool notb = a.probs[g.first].tb_off == NO_TB_OFF;  // (one problem a group)
+            // (one problem a group)
+            const bool notb = (GAP != GAP_DTW || VAR == VAR_CKPT) && a.probs[g.first].tb_off == NO_TB_OFF;
             bool mx = false;
             if constexpr (GAP == GAP_DTW && FORM == F_SERIES) mx = a.finite != nullptr && *a.finite != 0u;
             if (mx) {
@@ -1198,7 +1199,8 @@ static hipError_t go_fast(const LaunchSpec &s, const KArgs &a, hipStream_t st, i
 }
 
 template <int LOC, int DIR, int GAP, int FORM, int TR, int R, int SD, int VAR>
-__global__ __launch_bounds__(256) void pa_solve_kernel(KArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, VAR == VAR_CKPT ? 2 : 8))) void
+pa_solve_kernel(KArgs a) {
     extern __shared__ float lds_table[];
     if constexpr (FORM == F_TABLE) {
         const int n = a.K1 * a.K1;
@@ -1262,6 +1264,8 @@ static hipError_t dispatch_lg(const LaunchSpec &s, const KArgs &a, hipStream_t s
             if (s.var == VAR_VALUES) PA_GO_VAR(FORM, TR, R, SD, VAR_VALUES);                     \
         if constexpr (TR == TR_ONE && GAP != GAP_DTW && FORM != F_TABLE_G && FORM != F_SERIES)   \
             if (s.var == VAR_MAX) PA_GO_VAR(FORM, TR, R, SD, VAR_MAX);                           \
+        if constexpr (TR == TR_ONE && GAP == GAP_DTW)                                            \
+            if (s.var == VAR_CKPT) PA_GO_VAR(FORM, TR, R, SD, VAR_CKPT);                         \
         PA_GO_VAR(FORM, TR, R, SD, VAR_PLAIN);                                                   \
     } while (0)
     if constexpr (GAP == GAP_DTW) {
