@@ -484,49 +484,68 @@ int ilog2(int x) {
 #endif
 constexpr double STEP_OVERHEAD = PA_STEP_OVERHEAD;
 
-bool choose_layout(int64_t ls, int64_t lt, const std::vector<int> &Rs, double cap, int &L_out, int &R_out,
-                   double *cost_out = nullptr, double *serial_out = nullptr) {
-    double best_cost = 1e300, best_serial = 1e300;
-    int bL = 64, bR = Rs.back();
-    double fb_serial = 1e300, fb_cost = 1e300;
-    int fL = 64, fR = Rs.back();
-    int32_t lanes[16];  // lanes of R rows (one division per strip height, not per layout)
-    for (size_t q = 0; q < Rs.size(); q++) lanes[q] = int32_t((ls + Rs[q] - 1) / Rs[q]);
-    for (int lg = 0; lg <= 6; lg++) {
-        const int L = 1 << lg;
-        for (size_t q = 0; q < Rs.size(); q++) {
-            const int R = Rs[q];
-            const int32_t nst = (lanes[q] + L - 1) >> lg;
-            const double serial = double(nst) * double(lt + L - 1) * (STEP_OVERHEAD + R);
-            const double cost = serial * L;
-            if (serial < fb_serial || (serial == fb_serial && cost < fb_cost)) {
-                fb_serial = serial;
-                fb_cost = cost;
-                fL = L;
-                fR = R;
-            }
-            if (serial > cap) continue;
-            if (cost < best_cost || (cost == best_cost && serial < best_serial)) {
-                best_cost = cost;
-                best_serial = serial;
-                bL = L;
-                bR = R;
+struct Layout {
+    int L = 64, R = 0;
+    double cost = 0.0, serial = 0.0;
+    bool fit = false;
+};
+
+// Of the strip heights only the one with the least strips * (4 + R) matters for
+// each L, and a larger L only if it has fewer of those, whatever len_t: at most
+// seven candidates for a len_s, found once per len_s met (16,384 pairs of 100
+// to 150 x 200 to 400 over five heights: planned in 2.5 ms, 6.0 ms trying all for every pair).
+class Layouts {
+    struct Cand {
+        double column;  // serial cell units of a column: strips * (4 + R)
+        int32_t L, R;
+    };
+    struct Set {
+        int64_t ls = -1;
+        int n = 0;
+        Cand c[7];
+    };
+    const std::vector<int> &Rs;
+    std::vector<int32_t> slots;  // len_s -> its place in sets (colliding ones replaced); a power of two
+    std::vector<Set> sets;
+
+  public:
+    Layouts(const std::vector<int> &heights, int64_t n) : Rs(heights), slots(n > 64 ? 4096 : 1, -1) {}
+
+    Layout choose(int64_t ls, int64_t lt, double cap) {
+        int32_t &slot = slots[size_t(ls) & (slots.size() - 1)];
+        if (slot < 0) {
+            slot = int32_t(sets.size());
+            sets.emplace_back();
+        }
+        Set &set = sets[size_t(slot)];
+        if (set.ls != ls) {
+            set.ls = ls;
+            set.n = 0;
+            for (int lg = 0; lg <= 6; lg++) {
+                Cand best{1e300, 1 << lg, 0};
+                for (int R : Rs) {
+                    const int64_t lanes = (ls + R - 1) / R;
+                    const double column = double((lanes + best.L - 1) >> lg) * (STEP_OVERHEAD + R);
+                    if (column < best.column) {
+                        best.column = column;
+                        best.R = R;
+                    }
+                }
+                if (!set.n || best.column < set.c[set.n - 1].column) set.c[set.n++] = best;
             }
         }
+        Layout best, fall;
+        best.cost = fall.serial = 1e300;
+        for (int q = 0; q < set.n; q++) {
+            const Cand &c = set.c[q];
+            const double serial = c.column * double(lt + c.L - 1), cost = serial * c.L;
+            if (serial < fall.serial || (serial == fall.serial && cost < fall.cost)) fall = Layout{c.L, c.R, cost, serial, false};
+            if (serial <= cap && (cost < best.cost || (cost == best.cost && serial < best.serial)))
+                best = Layout{c.L, c.R, cost, serial, true};
+        }
+        return best.fit ? best : fall;
     }
-    const bool fit = best_cost != 1e300;
-    if (!fit) {
-        bL = fL;
-        bR = fR;
-        best_cost = fb_cost;
-        best_serial = fb_serial;
-    }
-    L_out = bL;
-    R_out = bR;
-    if (cost_out) *cost_out = best_cost;
-    if (serial_out) *serial_out = best_serial;
-    return fit;
-}
+};
 
 // Band mode for a problem no layout brings under the cap: strips of 64 * 8
 // rows run concurrently, each starting about 64 + BAND_PUB steps after the
@@ -583,6 +602,7 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
         for (int R : {4, 8, 16, 32})
             if (supported_R(job.form, job.tr, R)) Rs.push_back(R);
     }
+    Layouts layouts(Rs, n);
     // total wavefront time at the cheapest layouts (no cap) sets the cap:
     // an eighth of a SIMD's share of the work for the fast kernel, a
     // sixteenth for the general kernel (both measured best)
@@ -591,10 +611,7 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
     double total = 0.0;
     for (int64_t k = 0; k < n; k += stride) {
         if (ls[k] <= 0 || lt[k] <= 0) continue;
-        int L, R;
-        double cost = 0.0;
-        choose_layout(ls[k], lt[k], Rs, 1e300, L, R, &cost);
-        total += cost / 64.0 * double(std::min(stride, n - k));
+        total += layouts.choose(ls[k], lt[k], 1e300).cost / 64.0 * double(std::min(stride, n - k));
     }
 #ifndef PA_CAP_DIV
 #define PA_CAP_DIV 8.0
@@ -618,12 +635,10 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
             work = longest = waves = 0.0;
             for (int64_t k = 0; k < n; k += every) {
                 if (ls[k] <= 0 || lt[k] <= 0) continue;
-                int L, R;
-                double cost = 0.0, serial = 0.0;
-                choose_layout(ls[k], lt[k], Rs, c, L, R, &cost, &serial);
-                work += cost / 64.0 * double(every) / simds;
-                waves += L / 64.0 * double(every);
-                longest = std::max(longest, serial);
+                const Layout at = layouts.choose(ls[k], lt[k], c);
+                work += at.cost / 64.0 * double(every) / simds;
+                waves += at.L / 64.0 * double(every);
+                longest = std::max(longest, at.serial);
             }
             if (waves <= simds) return longest;
             return std::max(work, longest) + 0.5 * std::min(work, longest);
@@ -669,30 +684,22 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
         int nst;
     };
     std::vector<Cand> cands;  // problems the long mode could take
-    struct Layout {  // of the shapes met last (bags of short problems repeat theirs)
-        int32_t ls = 0, lt = 0, L = 0, R = 0;
-        double cost = 0.0, serial = 0.0;
-        bool fit = false;
+    struct Met {  // shapes met last (bags of short problems repeat theirs)
+        int32_t ls = -1, lt = -1;
+        Layout at;
     };
-    std::vector<Layout> memo(n >= 4096 ? 1024 : 1);
+    std::vector<Met> last_met(n >= 4096 ? 1024 : 1);
     for (int64_t k = 0; k < n; k++) {
-        int L = 64, R = Rs.back();
-        double serial = 0.0, cost = 0.0;
-        bool fit = true;
-        if (ls[k] > 0 && lt[k] > 0) {
-            Layout &m = memo[(size_t(ls[k]) * 31 + size_t(lt[k])) % memo.size()];
-            if (m.ls != ls[k] || m.lt != lt[k]) {
-                m.ls = ls[k];
-                m.lt = lt[k];
-                m.fit = choose_layout(ls[k], lt[k], Rs, cap, m.L, m.R, &m.cost, &m.serial);
-            }
-            L = m.L;
-            R = m.R;
-            cost = m.cost;
-            serial = m.serial;
-            fit = m.fit;
+        Met &met = last_met[(size_t(ls[k]) * 31 + size_t(lt[k])) & (last_met.size() - 1)];
+        if (met.ls != ls[k] || met.lt != lt[k]) {
+            met.ls = ls[k];
+            met.lt = lt[k];
+            met.at = ls[k] > 0 && lt[k] > 0 ? layouts.choose(ls[k], lt[k], cap) : Layout{1, Rs.front(), 0.0, 0.0, true};
         }
-        else { L = 1; R = Rs.front(); }
+        const Layout &at = met.at;
+        const int L = at.L, R = at.R;
+        const double serial = at.serial, cost = at.cost;
+        const bool fit = at.fit;
         const int64_t rps = int64_t(L) * R;
         const int nst = ls[k] > 0 && lt[k] > 0 ? int((ls[k] + rps - 1) / rps) : 0;
         if (ckpt && ckpt[k]) {

@@ -130,10 +130,54 @@ void fold_rule() {
     }
 }
 
+// The layout of a problem is the cheapest of all under the cap, or the one of
+// least serial time: the candidates kept per length against trying every one.
+void layouts() {
+    const std::vector<std::vector<int>> heights = {
+        {std::begin(FAST_RS), std::end(FAST_RS)}, {std::begin(FAST_RS_TABLE), std::end(FAST_RS_TABLE)},
+        {std::begin(FAST_RS_BINARY), std::end(FAST_RS_BINARY)}, {8}, {4, 8, 16, 32}};
+    uint64_t seed = 1;
+    auto draw = [&](int64_t most) {  // log-uniform, 1 .. most
+        seed = seed * 6364136223846793005ull + 1442695040888963407ull;
+        return int64_t(std::exp(double(seed >> 11) / 9007199254740992.0 * std::log(double(most) + 0.99)));
+    };
+    for (const auto &Rs : heights) {
+        Layouts kept(Rs, 1000);
+        for (int k = 0; k < 200000; k++) {
+            const int64_t ls = k % 7 ? draw(3000) : draw(200000), lt = draw(5000);
+            const double cap = k % 5 ? double(draw(1000000)) : 1e300;
+            double cost = 1e300, serial = 1e300, least = 1e300, least_cost = 1e300;
+            int L = 0, R = 0, fall_L = 0, fall_R = 0;
+            for (int l = 1; l <= 64; l *= 2)
+                for (int r : Rs) {
+                    const double s = double((ls + l * r - 1) / (l * r)) * double(lt + l - 1) * (STEP_OVERHEAD + r);
+                    if (s < least || (s == least && s * l < least_cost)) {
+                        least = s;
+                        least_cost = s * l;
+                        fall_L = l;
+                        fall_R = r;
+                    }
+                    if (s <= cap && (s * l < cost || (s * l == cost && s < serial))) {
+                        cost = s * l;
+                        serial = s;
+                        L = l;
+                        R = r;
+                    }
+                }
+            const Layout got = kept.choose(ls, lt, cap);
+            const bool fit = cost < 1e300;
+            expect(got.fit == fit && got.L == (fit ? L : fall_L) && got.R == (fit ? R : fall_R) &&
+                       got.cost == (fit ? cost : least_cost) && got.serial == (fit ? serial : least),
+                   "layout of " + std::to_string(ls) + " x " + std::to_string(lt) + " under " + std::to_string(cap));
+            if (bad > 5) return;
+        }
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"graph_key", graph_key}, {"wsb_extents", wsb_extents}, {"fold_rule", fold_rule}};
+    const std::map<std::string, std::function<void()>> checks = {{"graph_key", graph_key}, {"wsb_extents", wsb_extents}, {"fold_rule", fold_rule}, {"layouts", layouts}};
     if (argc != 2 || !checks.count(argv[1])) {
         std::printf("usage: host_checks CHECK\n");
         return 2;
