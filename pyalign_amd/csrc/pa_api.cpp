@@ -591,8 +591,10 @@ double long_band(int64_t lt, const Job &job) {
     return double(lt + WAVE - 1 + ((LONG_WAVES - 1) * long_dw(job.form) + 2) * LONG_T) * long_unit(job);
 }
 
+// lean: the caps and groups of least device memory (row buffers and group
+// descriptors) rather than of least time.
 Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, int simds,
-               const uint8_t *ckpt = nullptr, bool allow_band = true, bool allow_long = true) {
+               const uint8_t *ckpt = nullptr, bool allow_band = true, bool allow_long = true, bool lean = false) {
     std::vector<int> Rs;
     if (job.fast) {
         if (job.form == F_BINARY) Rs.assign(std::begin(FAST_RS_BINARY), std::end(FAST_RS_BINARY));
@@ -607,7 +609,7 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
     // an eighth of a SIMD's share of the work for the fast kernel, a
     // sixteenth for the general kernel (both measured best)
     // (of a large bag every few problems stand for all)
-    const int64_t stride = std::max<int64_t>(1, n / 4096);
+    const int64_t stride = lean ? 1 : std::max<int64_t>(1, n / 4096);
     double total = 0.0;
     for (int64_t k = 0; k < n; k += stride) {
         if (ls[k] <= 0 || lt[k] <= 0) continue;
@@ -628,7 +630,7 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
     // doublings.  On a sample of the problems.  16,384 semiglobal pairs of
     // 125 x 300: kernel 0.50 -> 0.29 ms; 1,039 DTW training pairs of up to 2,499
     // (a few more than SIMDs): 11.5 -> 9.2 ms.
-    {
+    if (!lean) {
         const int64_t every = std::max<int64_t>(1, n / 256);
         double work = 0.0, longest = 0.0, waves = 0.0;
         auto estimate = [&](double c) {
@@ -808,7 +810,7 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
             const double together = double(std::max<int32_t>(g.max_nst, items[p].nst)) *
                                     double(std::max<int64_t>(g.max_lt, items[p].lt) + L - 1);
             most = std::max(most, own);
-            if (cnt && together > 1.25 * most) break;
+            if (cnt && together > 1.25 * most && !lean) break;
             Prob pr{};
             pr.out = int32_t(items[p].k);
             pr.L = L;
@@ -1594,6 +1596,47 @@ void build_launches(pa_solver &s, const Job &job, const Input &in, const Plan &p
         specs.push_back(spec);
         largs.push_back(la);
     }
+}
+
+// The allocation-free solve's scratch: safe values, sink, queue tickets,
+// borders, table, problem and group descriptors, strip-boundary row buffer.
+struct NoallocLayout {
+    size_t safe, sink, queue, bs, bt, table, probs, groups, rowbuf, total = 0;
+    NoallocLayout(const pa_solver &s, const Input &in, const Plan &plan) {
+        auto take = [&](size_t bytes) {
+            const size_t here = total;
+            total = (total + bytes + 255) / 256 * 256;
+            return here;
+        };
+        safe = take(SAFE_FLOATS * 4);
+        sink = take(SINK_WORDS * 4);
+        queue = take(std::max<size_t>(plan.launches.size(), 1) * 4);
+        bs = take(s.border_s.size() * 4);
+        bt = take(s.border_t.size() * 4);
+        table = take(in.table.size() * 4);
+        probs = take(plan.probs.size() * sizeof(Prob));
+        groups = take(plan.groups.size() * sizeof(Group));
+        rowbuf = take(size_t(plan.rowbuf) * sizeof(float2));
+    }
+};
+
+// Its plan.  The fastest layouts may give a short problem few lanes and several
+// strips, and with them a row buffer (276,247 global pairs of up to 67 x 531 over
+// a table: 126 MB in all, and 30 MB with a strip each): where that does not fit,
+// the layouts of least memory, in the general kernel unless the job is a local
+// maximum over a table.
+Plan noalloc_plan(const pa_solver &s, const Input &in, Job &job, int cus) {
+    auto placed = [&](Plan plan) {
+        place_plan(plan, in, 0, false, 1);
+        return plan;
+    };
+    if (in.schedule == PA_SCHED_PLAIN) return placed(plan_plain(job, in.len_s, in.len_t, in.n));
+    // no band mode: its strips hand rows down through progress counters
+    // whose failure flag the host would have to read back
+    Plan plan = placed(plan_auto(job, in.len_s, in.len_t, in.n, cus * 4, nullptr, false));
+    if (NoallocLayout(s, in, plan).total <= NOALLOC_SCRATCH_BYTES) return plan;
+    job.fast = job.fast && job.form == F_TABLE && job.loc == LOC_LOCAL && job.dir == DIR_MAX;
+    return placed(plan_auto(job, in.len_s, in.len_t, in.n, cus * 4, nullptr, false, true, true));
 }
 
 // Everything that the arguments of a launch sequence are made from (see
@@ -2506,32 +2549,11 @@ int pa_solve_ragged_scores_noalloc(pa_solver *s, const pa_ragged *batch, int32_t
         int cus = 0;
         HIPCHK(noalloc_scratch(&base, &cus));
         if (!s->has_device) s->cus = cus;
-        // no band mode: its strips hand rows down through progress counters
-        // whose failure flag the host would have to read back
-        Plan plan = in.schedule == PA_SCHED_PLAIN ? plan_plain(job, in.len_s, in.len_t, n)
-                                                  : plan_auto(job, in.len_s, in.len_t, n, cus * 4, nullptr, false);
-        place_plan(plan, in, 0, false, 1);
-
-        // the scratch layout: safe values, sink, queue tickets, borders,
-        // table, problem and group descriptors, strip-boundary row buffer
-        size_t at = 0;
-        auto take = [&](size_t bytes) {
-            const size_t here = at;
-            at = (at + bytes + 255) / 256 * 256;
-            return here;
-        };
-        const size_t o_safe = take(SAFE_FLOATS * 4);
-        const size_t o_sink = take(SINK_WORDS * 4);
-        const size_t o_queue = take(std::max<size_t>(plan.launches.size(), 1) * 4);
-        const size_t o_bs = take(s->border_s.size() * 4);
-        const size_t o_bt = take(s->border_t.size() * 4);
-        const size_t o_table = take(in.table.size() * 4);
-        const size_t o_probs = take(plan.probs.size() * sizeof(Prob));
-        const size_t o_groups = take(plan.groups.size() * sizeof(Group));
-        const size_t o_rowbuf = take(size_t(plan.rowbuf) * sizeof(float2));
-        if (at > NOALLOC_SCRATCH_BYTES) {
+        const Plan plan = noalloc_plan(*s, in, job, cus);
+        const NoallocLayout to(*s, in, plan);
+        if (to.total > NOALLOC_SCRATCH_BYTES) {
             std::ostringstream e;
-            e << "the allocation-free solve needs " << at << " bytes of device scratch for this batch; it holds "
+            e << "the allocation-free solve needs " << to.total << " bytes of device scratch for this batch; it holds "
               << NOALLOC_SCRATCH_BYTES << " (use pa_solve_ragged_scores_device, or smaller batches)";
             fail(PA_EINVAL, e.str());
         }
@@ -2544,37 +2566,37 @@ int pa_solve_ragged_scores_noalloc(pa_solver *s, const pa_ragged *batch, int32_t
         auto put = [&](size_t off, const void *src, size_t bytes) {
             if (bytes) HIPCHK(hipMemcpyAsync(dev + off, src, bytes, hipMemcpyHostToDevice, st));
         };
-        put(o_safe, safe, sizeof(safe));
-        put(o_bs, s->border_s.data(), s->border_s.size() * 4);
-        put(o_bt, s->border_t.data(), s->border_t.size() * 4);
-        put(o_table, in.table.data(), in.table.size() * 4);
-        put(o_probs, plan.probs.data(), plan.probs.size() * sizeof(Prob));
-        put(o_groups, plan.groups.data(), plan.groups.size() * sizeof(Group));
+        put(to.safe, safe, sizeof(safe));
+        put(to.bs, s->border_s.data(), s->border_s.size() * 4);
+        put(to.bt, s->border_t.data(), s->border_t.size() * 4);
+        put(to.table, in.table.data(), in.table.size() * 4);
+        put(to.probs, plan.probs.data(), plan.probs.size() * sizeof(Prob));
+        put(to.groups, plan.groups.data(), plan.groups.size() * sizeof(Group));
 
         KArgs a;
         std::memset(&a, 0, sizeof(a));
-        a.probs = reinterpret_cast<const Prob *>(dev + o_probs);
-        a.groups = reinterpret_cast<const Group *>(dev + o_groups);
+        a.probs = reinterpret_cast<const Prob *>(dev + to.probs);
+        a.groups = reinterpret_cast<const Group *>(dev + to.groups);
         a.codes_s = in.codes_s;
         a.codes_t = in.codes_t;
-        a.table = reinterpret_cast<const float *>(dev + o_table);
+        a.table = reinterpret_cast<const float *>(dev + to.table);
         a.K1 = in.K1;
         a.dim = in.dim;
         a.eq = in.eq;
         a.ne = in.ne;
         a.dense = in.dense;
-        a.rowbuf = reinterpret_cast<float2 *>(dev + o_rowbuf);
-        a.border_s = reinterpret_cast<const float *>(dev + o_bs);
-        a.border_t = reinterpret_cast<const float *>(dev + o_bt);
-        a.safe = reinterpret_cast<const float *>(dev + o_safe);
-        a.sink = reinterpret_cast<uint32_t *>(dev + o_sink);
+        a.rowbuf = reinterpret_cast<float2 *>(dev + to.rowbuf);
+        a.border_s = reinterpret_cast<const float *>(dev + to.bs);
+        a.border_t = reinterpret_cast<const float *>(dev + to.bt);
+        a.safe = reinterpret_cast<const float *>(dev + to.safe);
+        a.sink = reinterpret_cast<uint32_t *>(dev + to.sink);
         a.go_s = s->go_s;
         a.ge_s = s->ge_s;
         a.go_t = s->go_t;
         a.ge_t = s->ge_t;
         a.scores = scores_device;
         a.val_layers = 1;
-        uint32_t *queue = reinterpret_cast<uint32_t *>(dev + o_queue);
+        uint32_t *queue = reinterpret_cast<uint32_t *>(dev + to.queue);
         std::vector<LaunchSpec> specs;
         std::vector<KArgs> largs;
         build_launches(*s, job, in, plan, a, queue, specs, largs);

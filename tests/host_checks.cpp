@@ -174,10 +174,42 @@ void layouts() {
     }
 }
 
+// The allocation-free solve: batches that fit its scratch in the layouts of
+// least memory are planned so where the fastest layouts do not fit.
+void noalloc_scratch_use() {
+    struct Batch {
+        uint32_t n, s, t;
+        int loc, form;
+    };
+    for (const Batch &b : {Batch{276247, 67, 531, LOC_GLOBAL, F_TABLE}, Batch{255324, 73, 355, LOC_GLOBAL, F_BINARY},
+                           Batch{318456, 44, 431, LOC_LOCAL, F_BINARY}}) {
+        pa_solver s;
+        s.opt.dir = PA_MAXIMIZE;
+        std::vector<int32_t> ls(b.n), lt(b.n);
+        std::vector<int64_t> off(b.n, 0);
+        for (uint32_t k = 0; k < b.n; k++) {
+            ls[k] = int32_t(1 + (k * 2654435761u >> 8) % b.s);
+            lt[k] = int32_t(1 + (k * 40503u >> 4) % b.t);
+        }
+        Input in{};
+        in.n = b.n;
+        in.form = b.form == F_TABLE ? PA_FORM_INDEXED : PA_FORM_BINARY;
+        in.schedule = PA_SCHED_AUTO;
+        in.len_s = ls.data();
+        in.len_t = lt.data();
+        in.off_s = in.off_t = off.data();
+        Job job{b.loc, DIR_MAX, GAP_AFF, b.form, TR_SCORE, true, true};
+        const Plan plan = noalloc_plan(s, in, job, 256);
+        const size_t bytes = NoallocLayout(s, in, plan).total;
+        expect(bytes <= NOALLOC_SCRATCH_BYTES, std::to_string(b.n) + " of up to " + std::to_string(b.s) + " x " +
+                                                   std::to_string(b.t) + ": " + std::to_string(bytes) + " bytes");
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"graph_key", graph_key}, {"wsb_extents", wsb_extents}, {"fold_rule", fold_rule}, {"layouts", layouts}};
+    const std::map<std::string, std::function<void()>> checks = {{"graph_key", graph_key}, {"wsb_extents", wsb_extents}, {"fold_rule", fold_rule}, {"layouts", layouts}, {"noalloc_scratch", noalloc_scratch_use}};
     if (argc != 2 || !checks.count(argv[1])) {
         std::printf("usage: host_checks CHECK\n");
         return 2;
