@@ -262,29 +262,42 @@ class Solution:
         return self._materialised()["traceback_as_edges"]
 
 
-class _Solved:
-    """The results of a solve that its Solutions read: scores, the paths and
-    alignments concatenated in problem order with their offsets, the algorithm
-    record, and lazy(k), problem k's Solution matrices."""
+class _Maps:
+    """The alignments of a solve: scores, and every s_to_t and t_to_s,
+    concatenated in problem order with their offsets."""
 
-    __slots__ = ("scores", "paths", "path_at", "s_to_t", "s_at", "t_to_s", "t_at", "algorithm", "lazy")
+    __slots__ = ("scores", "s_to_t", "s_at", "t_to_s", "t_at")
+
+    def s_map(self, k):
+        return self.s_to_t[self.s_at[k]:self.s_at[k + 1]]
+
+    def t_map(self, k):
+        return self.t_to_s[self.t_at[k]:self.t_at[k + 1]]
+
+
+class _Solved:
+    """The results of a solve that its Solutions read: the alignments and their
+    scores, the paths (concatenated like them), the algorithm record, and
+    lazy(k), problem k's Solution matrices."""
+
+    __slots__ = ("maps", "scores", "paths", "path_at", "algorithm", "lazy")
 
 
 class _BagSolution(Solution):
-    """Problem k's Solution of a solve, its arrays cut out on first use; it also
-    reads like its own Alignment (s_to_t, t_to_s), so that a Solution of
-    solve.py needs no further object for one.  No instance dict: Python's
-    collector has one object per problem to visit (4,096 Solutions of 100 x 100
-    alignments, built and read: 17 ms with eager objects and dicts, 7 ms)."""
+    """Problem k's Solution of a solve, its arrays cut out on first use; an
+    Alignment of solve.py takes the maps and _k instead of one made here.  No
+    instance dict: Python's collector has one object per problem to visit (4,096
+    Solutions of 100 x 100 alignments, built and read: 17 ms with eager objects
+    and dicts, 7 ms)."""
 
-    __slots__ = ("_solved", "_k", "_cut_path", "_cut_s", "_cut_t", "_made", "_made_lazy")
+    __slots__ = ("_solved", "_k", "_cut_path", "_made", "_made_lazy")
 
     _max_degree_1 = True
 
     def __init__(self, solved, k):
         self._solved = solved
         self._k = k
-        self._cut_path = self._cut_s = self._cut_t = self._made = self._made_lazy = None
+        self._cut_path = self._made = self._made_lazy = None
 
     @property
     def score(self):
@@ -298,23 +311,10 @@ class _BagSolution(Solution):
         return self._cut_path
 
     @property
-    def s_to_t(self):
-        if self._cut_s is None:
-            at = self._solved.s_at
-            self._cut_s = self._solved.s_to_t[at[self._k]:at[self._k + 1]]
-        return self._cut_s
-
-    @property
-    def t_to_s(self):
-        if self._cut_t is None:
-            at = self._solved.t_at
-            self._cut_t = self._solved.t_to_s[at[self._k]:at[self._k + 1]]
-        return self._cut_t
-
-    @property
     def alignment(self):
         if self._made is None:
-            self._made = Alignment(self.score, self.s_to_t, self.t_to_s)
+            maps = self._solved.maps
+            self._made = Alignment(self.score, maps.s_map(self._k), maps.t_map(self._k))
         return self._made
 
     @property
@@ -489,10 +489,13 @@ class Solver:
             b = [0] + np.cumsum(r.len_t).tolist()
             return tuple([Alignment(x, s2t[a[k]:a[k + 1]], t2s[b[k]:b[k + 1]]) for k, x in enumerate(scores.tolist())])
 
+        # (Solutions keep `lazy`, which keeps the lengths but no result handle alive)
+        all_s, all_t = r.len_s, r.len_t
+
         def lazy(k):
             if one is None:
                 return None
-            a, b = int(r.len_s[k]), int(r.len_t[k])  # the closure keeps no result handle alive
+            a, b = int(all_s[k]), int(all_t[k])
 
             def make():
                 form, payload = one(k)
@@ -519,16 +522,17 @@ class Solver:
             return [0] + np.cumsum(x).tolist()
 
         v = _Solved()
-        v.scores = scores.tolist()
+        v.maps = m = _Maps()
+        v.scores = m.scores = scores.tolist()
+        m.s_to_t, m.s_at = s2t, offsets(r.len_s)
+        m.t_to_s, m.t_at = t2s, offsets(r.len_t)
         v.paths, v.path_at = uv, offsets(np.maximum(lens, 0))
-        v.s_to_t, v.s_at = s2t, offsets(r.len_s)
-        v.t_to_s, v.t_at = t2s, offsets(r.len_t)
         v.algorithm = _algorithm_for(self._opts)
         v.lazy = lazy
         if (lens >= 0).all():
             return tuple([_BagSolution(v, k) for k in range(n)])
-        return tuple([Solution(None, None, None, v.algorithm, lazy=lazy(k)) if m < 0 else _BagSolution(v, k)
-                      for k, m in enumerate(lens.tolist())])
+        return tuple([Solution(None, None, None, v.algorithm, lazy=lazy(k)) if x < 0 else _BagSolution(v, k)
+                      for k, x in enumerate(lens.tolist())])
 
     def _matrices(self, form, ls, lt, payload):
         """Solve one problem again with its DP matrices kept."""

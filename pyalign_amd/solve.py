@@ -51,10 +51,10 @@ class Solution:
     def alignment(self):
         if self._alignment is None:
             core = self._solution
-            if not isinstance(core, algorithm._BagSolution):  # (one reads like its own alignment)
-                core = core.alignment
-            if core is not None:
-                self._alignment = Alignment(self._problem, self._solver, core)
+            if isinstance(core, algorithm._BagSolution):
+                self._alignment = Alignment(self._problem, self._solver, core._solved.maps, core._k)
+            elif core.alignment is not None:
+                self._alignment = Alignment(self._problem, self._solver, core.alignment)
         return self._alignment
 
     @property
@@ -87,14 +87,18 @@ class Solution:
 
 
 class Alignment:
-    """A specific alignment that is part of a solution."""
+    """A specific alignment that is part of a solution.  `alignment` is the core
+    solver's, or with `k` the alignments of a bag (of which this one keeps no
+    more than the maps alive), cut out on first use."""
 
-    __slots__ = ("_problem", "_solver", "_alignment", "__dict__", "__weakref__")
+    __slots__ = ("_problem", "_solver", "_alignment", "_k", "_s_to_t", "_t_to_s", "__dict__", "__weakref__")
 
-    def __init__(self, problem, solver, alignment):
+    def __init__(self, problem, solver, alignment, k=None):
         self._problem = problem
         self._solver = solver
         self._alignment = alignment
+        self._k = k
+        self._s_to_t = self._t_to_s = None
 
     @property
     def problem(self):
@@ -106,15 +110,21 @@ class Alignment:
 
     @property
     def score(self):
-        return self._alignment.score
+        return self._alignment.score if self._k is None else self._alignment.scores[self._k]
 
     @property
     def s_to_t(self):
-        return self._alignment.s_to_t
+        if self._s_to_t is None:
+            core, k = self._alignment, self._k
+            self._s_to_t = core.s_to_t if k is None else core.s_to_t[core.s_at[k]:core.s_at[k + 1]]
+        return self._s_to_t
 
     @property
     def t_to_s(self):
-        return self._alignment.t_to_s
+        if self._t_to_s is None:
+            core, k = self._alignment, self._k
+            self._t_to_s = core.t_to_s if k is None else core.t_to_s[core.t_at[k]:core.t_at[k + 1]]
+        return self._t_to_s
 
     @cached_property
     def edges(self):
