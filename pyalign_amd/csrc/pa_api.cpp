@@ -135,8 +135,11 @@ namespace {
 
 // Pinned host buffers of results, kept by a solver and its results: a
 // result's buffer is written by one device copy and goes back when the result
-// is freed (at most two wait for reuse).
+// is freed.  At most two wait for reuse, and together at most 128 MiB (4,096
+// results of 100 x 100 take 5 MB; a larger buffer costs 25 us a MiB to allocate
+// anew, little beside the solve that fills it).
 struct PinPool {
+    static constexpr size_t IDLE_BYTES = size_t(128) << 20;
     struct Buf {
         char *p = nullptr;
         size_t cap = 0;
@@ -163,16 +166,25 @@ struct PinPool {
     }
     void give(Buf b) {
         if (!b.p) return;
+        Buf over[3];  // the smallest while there are too many, the largest while they are too large
+        size_t n = 0;
         {
             std::lock_guard<std::mutex> lock(mu);
             idle.push_back(b);
-            if (idle.size() <= 2) return;
-            auto least = std::min_element(idle.begin(), idle.end(),
-                                          [](const Buf &x, const Buf &y) { return x.cap < y.cap; });
-            b = *least;
-            idle.erase(least);
+            auto smaller = [](const Buf &x, const Buf &y) { return x.cap < y.cap; };
+            auto drop = [&](std::vector<Buf>::iterator it) {
+                over[n++] = *it;
+                idle.erase(it);
+            };
+            if (idle.size() > 2) drop(std::min_element(idle.begin(), idle.end(), smaller));
+            while (!idle.empty() && held() > IDLE_BYTES) drop(std::max_element(idle.begin(), idle.end(), smaller));
         }
-        (void)hipHostFree(b.p);
+        while (n) (void)hipHostFree(over[--n].p);
+    }
+    size_t held() const {
+        size_t sum = 0;
+        for (const Buf &b : idle) sum += b.cap;
+        return sum;
     }
 };
 

@@ -206,10 +206,32 @@ void noalloc_scratch_use() {
     }
 }
 
+// Idle result buffers: two at most, the larger ones, within the pool's bytes.
+// (The buffers here are no memory; the pool only ever hands them on.)
+void pin_pool() {
+    const size_t MB = size_t(1) << 20;
+    auto kept = [&](std::vector<size_t> given) {
+        auto *pool = new PinPool;
+        for (size_t q = 0; q < given.size(); q++)
+            pool->give(PinPool::Buf{reinterpret_cast<char *>(4096 * (q + 1)), given[q] * MB});
+        std::multiset<size_t> caps;
+        for (const PinPool::Buf &b : pool->idle) caps.insert(b.cap / MB);
+        expect(pool->held() <= PinPool::IDLE_BYTES, "more bytes idle than the pool may hold");
+        pool->idle.clear();
+        delete pool;
+        return caps;
+    };
+    expect(kept({1, 2}) == std::multiset<size_t>{1, 2}, "two small buffers");
+    expect(kept({5, 1, 2}) == std::multiset<size_t>{2, 5}, "the smallest of three goes");
+    expect(kept({100, 100}) == std::multiset<size_t>{100}, "two that are too large together");
+    expect(kept({3, 1000}) == std::multiset<size_t>{3}, "one that is too large alone");
+    expect(kept({100, 40, 50}) == std::multiset<size_t>{40, 50}, "the largest goes where two are too large");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"graph_key", graph_key}, {"wsb_extents", wsb_extents}, {"fold_rule", fold_rule}, {"layouts", layouts}, {"noalloc_scratch", noalloc_scratch_use}};
+    const std::map<std::string, std::function<void()>> checks = {{"graph_key", graph_key}, {"wsb_extents", wsb_extents}, {"fold_rule", fold_rule}, {"layouts", layouts}, {"noalloc_scratch", noalloc_scratch_use}, {"pin_pool", pin_pool}};
     if (argc != 2 || !checks.count(argv[1])) {
         std::printf("usage: host_checks CHECK\n");
         return 2;
