@@ -330,11 +330,14 @@ struct pa_result {
     // from off[k], off[n + 1 + k] and off[2 (n + 1) + k] on: path points, s, t)
     std::shared_ptr<PinPool> pool;
     PinPool::Buf pin;
+    bool copying = false;  // the buffer's copy is on its way on `stream` (a solve that fails later leaves it so)
+    hipStream_t stream = nullptr;
     std::vector<int64_t> off;
     const float *scores = nullptr;
     const int32_t *path_len = nullptr;
     const char *s_to_t = nullptr, *t_to_s = nullptr, *paths = nullptr;
     ~pa_result() {
+        if (copying) (void)hipStreamSynchronize(stream);
         if (pool) pool->give(pin);
     }
     int width() const { return index_bits == 16 ? 2 : 4; }
@@ -1196,6 +1199,8 @@ void fetch_results(pa_solver &s, hipStream_t st, pa_result &r, const float *scor
         r.paths = r.pin.p + at_p;
     }
     r.scores = reinterpret_cast<const float *>(r.pin.p);
+    r.stream = st;
+    r.copying = true;
     HIPCHK(hipMemcpyAsync(r.pin.p, src, bytes, hipMemcpyDeviceToHost, st));
 }
 
@@ -1474,6 +1479,7 @@ void run_wsb(pa_solver &s, const Input &in, const Job &job, std::unique_ptr<pa_r
         if (job.tr == TR_ALL) r->iters.resize(size_t(n));
     }
     HIPCHK(hipStreamSynchronize(st));
+    r->copying = false;
     float ms = 0.0f;
     HIPCHK(hipEventElapsedTime(&ms, s.ev0, s.ev1));
     s.last_ms = ms;
@@ -2052,6 +2058,7 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
         if (job.tr == TR_ALL) r->iters.resize(static_cast<size_t>(n));
     }
     HIPCHK(hipStreamSynchronize(st));
+    r->copying = false;
     check_band(s);
     float ms = 0.0f;
     HIPCHK(hipEventElapsedTime(&ms, s.ev0, s.ev1));
