@@ -45,12 +45,12 @@ __device__ __forceinline__ float opt(float a, float b) {
 
 // Traceback flags without lane masks: the sign of lead(a, b) says that b is
 // strictly better than a (their difference is exact in sign, and +0 for equal
-// values; two infinities of one sign give a NaN of either sign, so the caller
-// keeps them out), and push_sign shifts it into a
-// word with one v_alignbit_b32.  A compare, its 64-bit mask in scalar
-// registers and a select of a constant cost as many instructions and the wait
-// states between mask and select (38 s_nop in an 8-cell Gotoh step; 2,048 local
-// pairs, the general kernel's part: 1.43 -> 1.19 ms).
+// values; two infinities of one sign give a NaN, whose sign is set here: the
+// callers keep them out), and push_sign shifts it into a word with one
+// v_alignbit_b32.  A compare, its 64-bit mask in scalar registers and a select
+// of a constant cost as many instructions and the wait states between mask and
+// select (38 s_nop in an 8-cell Gotoh step; 2,048 local pairs, the general
+// kernel's part: 1.43 -> 1.19 ms).
 template <int DIR>
 __device__ __forceinline__ float lead(float a, float b) {
     return DIR == DIR_MAX ? a - b : b - a;
@@ -380,7 +380,7 @@ __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, cons
             constexpr bool KEEPV = KM == 1;  // cell values stored (a.dvals set)
             // no traceback stored (a checkpointed forward's group): the codes are not computed
             constexpr bool NOTB = KM == 2 || KM == 4;
-            // min / max folds, codes from equality tests (DTW: finite series)
+            // min / max folds, codes from signs (DTW: series up to SERIES_MOST)
             constexpr bool MXF = KM >= 3;
             const int j = s - l;
             const int tsym = cur.sym;
@@ -666,10 +666,10 @@ __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, cons
         // carries no per-cell test: 0 codes stored, 1 codes and cell values
         // (a.dvals; kernels of their own, VAR_VALUES), 2 neither (the groups of
         // a checkpointed forward keep strip rows only; their folds keep their
-        // order, their codes go; DTW: VAR_CKPT); 3 and 4 as 0 and 2 with min / max folds (DTW
-        // over finite series; alignment over tables and binary symbols in
-        // kernels of their own, VAR_MAX: a kernel holds the registers of its
-        // largest loop, 256 and a wave per SIMD where these shared one)
+        // order, their codes go; DTW: VAR_CKPT); 3 and 4 as 0 and 2 with min /
+        // max folds (DTW over series up to SERIES_MOST; alignment in kernels of
+        // their own, VAR_MAX: a kernel holds the registers of its largest loop,
+        // 256 and a wave per SIMD where these shared one)
         using Gen = integral_constant<bool, false>;
         auto watched = [&] { return WATCH && __any(odd_value); };  // (the sweep is for nothing)
         auto sweep = [&](auto kv) {
@@ -833,8 +833,8 @@ __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, cons
 // ---------------------------------------------------------------------------
 // The score kernel: score-only alignment over an LDS table or binary symbols
 // where max / min folds return the strict folds' bits (local maximisation
-// over a NaN-free table, see the file comment; elsewhere similarities finite
-// and no candidate -0, checked on the host).  Same decomposition as
+// over a NaN-free table, see the file comment; elsewhere by the host's
+// folds_max).  Same decomposition as
 // solve_group with the traceback and seed positions removed; one kernel
 // serves every strip height from one queue.
 //

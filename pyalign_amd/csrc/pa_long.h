@@ -81,12 +81,11 @@ __device__ __forceinline__ constexpr int long_ooff(int w) {
 
 // MX: the strict compare-and-select of every candidate fold done as max
 // (maximising) or min; the host chooses it where it returns the same bits:
-// similarities finite and never -0, and (maximising global problems) gap
-// costs above zero, so that no candidate is -0 or NaN (x + y is -0 only when
-// both are -0) and max / min keep the strict fold's value.  The strict fold
-// then chooses the first candidate in push order equal to that value, so
-// traceback codes come from sign tests beside the value chain instead
-// of lengthening it.
+// no candidate is -0 or NaN (x + y is -0 only when both are -0) and no value
+// infinite (folds_max in pa_api.cpp), so that max / min keep the strict fold's
+// value.  The strict fold then chooses the first candidate in push order equal
+// to that value, so traceback codes come from sign tests beside the value chain
+// instead of lengthening it.
 template <int LOC, int DIR, int GAP, int FORM, int TR, bool MX>
 __global__ __launch_bounds__((LONG_WAVES + 1) * WAVE) void pa_long_kernel(KArgs a, LongArgs la) {
     static_assert(LONG_R == 1, "one row per lane");

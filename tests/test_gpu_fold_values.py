@@ -24,14 +24,12 @@ VALUES = {"infinite open": (("affine", INF, 1), (2.0, -1.0)),
           "huge costs": (("affine", 1e30, 1e30), (1e30, -1e30))}
 
 
-@pytest.mark.parametrize("loc", list(LOCS))
-@pytest.mark.parametrize("values", list(VALUES))
+# (global, infinite linear: 0 * inf makes the corner of the borders NaN)
+@pytest.mark.parametrize("loc,values", [(x, v) for x in LOCS for v in VALUES if (x, v) != ("global", "infinite linear")])
 @pytest.mark.parametrize("direction", ["maximize", "minimize"])
 @pytest.mark.parametrize("form", ["indexed", "binary"])
 def test_values(loc, values, direction, form):
     gap, (eq, ne) = VALUES[values]
-    if loc == "global" and gap == ("linear", INF):
-        pytest.skip("0 * inf: a NaN corner")
     if direction == "minimize":
         eq, ne = -eq, -ne
     rng = np.random.default_rng(zlib.crc32(repr((loc, values, direction, form)).encode()))

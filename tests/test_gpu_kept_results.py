@@ -48,7 +48,7 @@ def test_an_alignment_keeps_the_maps_only():
     core = [x._solution.alignment for x in solutions]  # (the core solver's own)
     del solutions
     gc.collect()
-    assert not [x for x in gc.get_objects() if isinstance(x, (algorithm._Solved, algorithm._BagSolution))]
+    assert not [x for x in gc.get_objects() if type(x) in (algorithm._Solved, algorithm._BagSolution)]
     for al, own, (score, path, s_to_t) in zip(alignments, core, want):
         assert al.score == score == own.score and al.s_to_t is al.s_to_t and al.t_to_s is al.t_to_s
         assert np.array_equal(al.s_to_t, s_to_t) and np.array_equal(own.s_to_t, s_to_t)
