@@ -1664,7 +1664,9 @@ Plan noalloc_plan(const pa_solver &s, const Input &in, Job &job, int cus) {
 std::string launch_key(const Job &job, const Plan &plan, const std::vector<LaunchSpec> &specs,
                        const std::vector<KArgs> &largs, const KArgs &a, const LongArgs &la, int long_grid,
                        const int32_t *band_words, int64_t finite_nx, int64_t finite_ny) {
-    std::string key(reinterpret_cast<const char *>(specs.data()), specs.size() * sizeof(LaunchSpec));
+    std::string key;
+    key.reserve(specs.size() * sizeof(LaunchSpec) + (largs.size() + 1) * sizeof(KArgs) + sizeof(la) + 256);
+    key.append(reinterpret_cast<const char *>(specs.data()), specs.size() * sizeof(LaunchSpec));
     key.append(reinterpret_cast<const char *>(largs.data()), largs.size() * sizeof(KArgs));
     key.append(reinterpret_cast<const char *>(&a), sizeof(a));
     key.append(reinterpret_cast<const char *>(&la), sizeof(la));
