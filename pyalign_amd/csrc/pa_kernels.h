@@ -861,8 +861,8 @@ __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, cons
 // one address add (K1^2 * Kc * 8 bytes: 70,560 for 20 symbols and the pad).
 //
 // Bound by VALU issue.  Kernel times on one MI355X: 65,536 local Gotoh pairs of
-// 50 to 2,000 over a table 3.7 ms; 16,384 global affine pairs of 50 to 1,000
-// 0.5 ms (the general kernel's strict folds with long mode 8.6 ms); 16,384
+// 50 to 2,000 over a table 3.5 ms; 16,384 global affine pairs of 50 to 1,000
+// 0.53 ms (the general kernel's strict folds with long mode 8.6 ms); 16,384
 // semiglobal affine pairs of 125 x 300 binary symbols 0.29 ms (0.51 ms).
 // ---------------------------------------------------------------------------
 enum { SRC_TABLE = 0, SRC_PAIR = 1, SRC_BINARY = 2 };

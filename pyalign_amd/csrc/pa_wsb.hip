@@ -26,9 +26,10 @@
 // that solve the next anti-diagonal, so a launch's critical path is two folds
 // and the solve.
 //
-// The bound of (1) is VALU issue, 1.5 instructions per candidate, and of (2)
-// 1,300 instructions per four blocks; a launch takes at least 8 us (dependent
-// loads and the serial solve).  Measured: 1,024 pairs of 100 to 300 (local, 20
+// (1) takes 1.5 instructions per candidate and (2) 1,300 per four blocks, and a
+// launch at least 8 us (dependent loads and the serial solve): that, and each
+// launch's longest workgroup, bounds both below (0.31 VALU instructions per SIMD
+// in four cycles over the first's launches).  Measured: 1,024 pairs of 100 to 300 (local, 20
 // symbols) 1.6 ms and their paths 0.18 ms, one global pair of 1,200 x 1,000
 // 1.6 ms (3.5 ms without carried sums) and 0.23 ms.  The cell-by-cell kernel
 // (pa_wsb_kernel: two 4-byte loads, an add, a compare and two selects per
