@@ -701,6 +701,7 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
         int nst;
     };
     std::vector<Cand> cands;  // problems the long mode could take
+    double other = 0.0;       // the longest of the others
     struct Met {  // shapes met last (bags of short problems repeat theirs)
         int32_t ls = -1, lt = -1;
         Layout at;
@@ -728,16 +729,19 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
             items[size_t(k)] = Item{k, 0, 0, 0, 0, 0.0, false};
             continue;
         }
+        // (at least one strip per compute wave of a workgroup: shorter
+        // problems leave its waves idle)
+        bool could = false;
         if (!fit && long_ok && serial > crit) {
             int nl = 0;
             const double sl = long_serial(ls[k], lt[k], job, &nl);
-            // (at least one strip per compute wave of a workgroup: shorter
-            // problems leave its waves idle)
-            if (nl >= LONG_WAVES && sl < serial) {
+            could = nl >= LONG_WAVES;
+            if (could) {
                 const double lc = double((nl + LONG_WAVES - 1) / LONG_WAVES) * long_band(lt[k], job);
                 cands.push_back(Cand{k, serial, cost / 64.0, sl, lc, nl});
             }
         }
+        if (!could) other = std::max(other, serial);
         if (!fit && band_ok && !long_ok && serial > crit) {
             int nb = 0;
             const int bR = band_R(job.form, job.tr);
@@ -758,17 +762,20 @@ Plan plan_auto(const Job &job, const int32_t *ls, const int32_t *lt, int64_t n, 
     // last as long as their longest problem or their work spread over the GPU
     // (SIMDs; a band per CU), one after the other.  (16,384 global pairs of 50
     // to 1,000, score only: every problem above a quarter of a SIMD's share
-    // 8.6 ms, none 0.65 ms.)
+    // 8.6 ms, none 0.65 ms.)  A problem that alone would be no faster in long
+    // mode is one it could take too: left behind, it would be a launch of its own
+    // after the others (31 binary pairs of about 1,492 x 300 to 846, score only:
+    // six left behind 0.46 ms, none 0.22 ms).
     if (!cands.empty()) {
         std::stable_sort(cands.begin(), cands.end(), [](const Cand &a, const Cand &b) { return a.serial > b.serial; });
         double rest = total, long_max = 0.0, long_sum = 0.0;
-        double best = std::max(cands[0].serial, total / simds);
+        double best = std::max(std::max(cands[0].serial, other), total / simds);
         size_t take = 0;
         for (size_t q = 0; q < cands.size(); q++) {
             rest -= cands[q].cost;
             long_max = std::max(long_max, cands[q].long_serial);
             long_sum += cands[q].long_cost;
-            const double next = q + 1 < cands.size() ? cands[q + 1].serial : (int64_t(q) + 1 < n ? crit : 0.0);
+            const double next = std::max(q + 1 < cands.size() ? cands[q + 1].serial : 0.0, other);
             const double t = std::max(long_max, long_sum / (double(simds) / 4.0)) +
                              std::max(next, std::max(rest, 0.0) / simds);
             if (t < best) {

@@ -228,10 +228,34 @@ void pin_pool() {
     expect(kept({100, 40, 50}) == std::multiset<size_t>{40, 50}, "the largest goes where two are too large");
 }
 
+// Bags of a few long pairs: none is left behind for a launch of its own after
+// the long mode's; short pairs beside them are.
+void long_choice() {
+    struct Bag {
+        int form;
+        std::vector<std::pair<int, int>> shapes;
+        int longs;
+    };
+    for (const Bag &b : {Bag{F_BINARY, {{726, 297}, {766, 889}}, 2}, Bag{F_BINARY, {{229, 432}, {244, 500}, {234, 147}}, 3},
+                         Bag{F_BINARY, {{1492, 790}, {1492, 307}, {1492, 462}, {1492, 366}, {1492, 846}}, 5},
+                         Bag{F_TABLE, {{1571, 576}, {956, 237}, {1270, 1093}, {347, 490}}, 4},
+                         Bag{F_TABLE, {{5000, 4000}, {20, 30}}, 1}, Bag{F_TABLE, {{20, 30}, {50, 60}}, 0}}) {
+        std::vector<int32_t> ls, lt;
+        for (const auto &x : b.shapes) {
+            ls.push_back(x.first);
+            lt.push_back(x.second);
+        }
+        const Plan plan = plan_auto(Job{LOC_GLOBAL, DIR_MAX, GAP_AFF, b.form, TR_SCORE, true, true}, ls.data(), lt.data(),
+                                    int64_t(ls.size()), 1024);
+        expect(plan.n_long == b.longs, std::to_string(ls[0]) + " x " + std::to_string(lt[0]) + " and others: " +
+                                           std::to_string(plan.n_long) + " of " + std::to_string(ls.size()) + " long");
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"graph_key", graph_key}, {"wsb_extents", wsb_extents}, {"fold_rule", fold_rule}, {"layouts", layouts}, {"noalloc_scratch", noalloc_scratch_use}, {"pin_pool", pin_pool}};
+    const std::map<std::string, std::function<void()>> checks = {{"graph_key", graph_key}, {"wsb_extents", wsb_extents}, {"fold_rule", fold_rule}, {"layouts", layouts}, {"noalloc_scratch", noalloc_scratch_use}, {"pin_pool", pin_pool}, {"long_choice", long_choice}};
     if (argc != 2 || !checks.count(argv[1])) {
         std::printf("usage: host_checks CHECK\n");
         return 2;

@@ -9,7 +9,7 @@ import pytest
 from pyalign_amd import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-CHECKS = ["graph_key", "wsb_extents", "fold_rule", "layouts", "noalloc_scratch", "pin_pool"]
+CHECKS = ["graph_key", "wsb_extents", "fold_rule", "layouts", "noalloc_scratch", "pin_pool", "long_choice"]
 
 
 @pytest.fixture(scope="session")
