@@ -1923,13 +1923,14 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
     // A launch sequence repeated with identical arguments (same shapes, same
     // buffers) is captured once as a hipGraph and replayed; the kernels read
     // the plan and inputs uploaded just before, so a replay sees new data.
-    const std::string gkey = launch_key(job, plan, specs, largs, a, la, long_grid, band_words, finite_nx, finite_ny);
+    // Graphs are captured on the solver's own stream only (a caller's stream
+    // may be the null stream, or under a capture of its own).
+    const bool graphs = s.use_graphs && !s.external_stream;
+    std::string gkey;
+    if (graphs) gkey = launch_key(job, plan, specs, largs, a, la, long_grid, band_words, finite_nx, finite_ny);
 
     HIPCHK(hipEventRecord(s.ev0, st));
     hipError_t le = hipSuccess;
-    // graphs are captured on the solver's own stream only (a caller's stream
-    // may be the null stream, or under a capture of its own)
-    const bool graphs = s.use_graphs && !s.external_stream;
     if (graphs && s.graph_exec && gkey == s.graph_key) {
         le = hipGraphLaunch(s.graph_exec, st);
     } else if (graphs && gkey == s.prev_key) {
@@ -1954,7 +1955,7 @@ void run(pa_solver &s, const Input &in, std::unique_ptr<pa_result> *result, floa
     } else {
         le = enqueue();
     }
-    s.prev_key = gkey;
+    s.prev_key = std::move(gkey);
     if (le != hipSuccess) {
         std::ostringstream m;
         m << "kernel launch failed (loc " << job.loc << " dir " << job.dir << " gap " << job.gap << " form "
