@@ -1594,23 +1594,35 @@ void build_launches(pa_solver &s, const Job &job, const Input &in, const Plan &p
                 spec.lds_bytes = pair_bytes;
             }
         }
-        const std::vector<int> okey = {spec.loc, spec.dir, spec.gap, spec.form, spec.tr, spec.R,
-                                       int(spec.fastmax), int(spec.lds_bytes), spec.pair, in.dim, spec.var};
+        auto resident = [&](int block) {  // waves per CU of workgroups of that size
+            spec.block = block;
+            const std::vector<int> okey = {spec.loc, spec.dir, spec.gap, spec.form, spec.tr, spec.R, int(spec.fastmax),
+                                           int(spec.lds_bytes), spec.pair, in.dim, spec.var, block};
+            for (auto &e : s.occ_cache)
+                if (e.first == okey) return e.second;
+            const int waves = std::max(1, occupancy_waves(spec, in.dim));
+            s.occ_cache.push_back({okey, waves});
+            return waves;
+        };
+        // The score kernel's large workgroups only where the groups fill every
+        // CU with them; fewer groups spread over more, smaller workgroups, unless
+        // their LDS (a pair table each) keeps some of those from running at
+        // once: their groups would wait for a whole launch of the others
+        // (17,667 global pairs of about 43 x 850, 2,274 groups: workgroups of 256
+        // 0.30 ms, of 512 0.19 ms).
+        const int64_t n_groups = g1 - g0;
         int waves_per_cu = 0;
-        for (auto &e : s.occ_cache)
-            if (e.first == okey) waves_per_cu = e.second;
-        if (!waves_per_cu) {
-            waves_per_cu = std::max(1, occupancy_waves(spec, in.dim));
-            s.occ_cache.push_back({okey, waves_per_cu});
+        if (fastmax && n_groups >= int64_t(s.cus) * (FAST_BLOCK / WAVE)) {
+            waves_per_cu = resident(FAST_BLOCK);
+        } else {
+            waves_per_cu = resident(256);
+            if (fastmax && int64_t(s.cus) * waves_per_cu < n_groups) waves_per_cu = resident(512);
         }
         // Band-mode strips wait for the strips above them: a third wave per SIMD
         // (DTW's traceback build has the registers for it) mostly polls and
         // slows the other two.  1,039 DTW pairs of 500 to 2,000, nearly all in
         // strips: two waves 5.0 ms, three 5.8 ms.
         if (!fastmax && int64_t(plan.band_probs.size()) > plan.n_long) waves_per_cu = std::min(waves_per_cu, 8);
-        // the fast kernel's large workgroups only where the groups fill every
-        // CU with them; fewer groups spread over more, smaller workgroups
-        spec.block = fastmax && R == 0 && int64_t(g1 - g0) >= int64_t(s.cus) * (FAST_BLOCK / WAVE) ? FAST_BLOCK : 256;
         const int wpb = spec.block / WAVE;  // waves per workgroup
         const int64_t wg_needed = (int64_t(g1 - g0) + wpb - 1) / wpb;
         spec.grid = int(std::max<int64_t>(1, std::min<int64_t>(wg_needed, int64_t(s.cus) * std::max(1, waves_per_cu / wpb))));

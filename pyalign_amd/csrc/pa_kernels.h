@@ -1174,14 +1174,13 @@ __global__ __launch_bounds__(FAST_BLOCK) void pa_fast_kernel(KArgs a) {
 template <int LOC, int DIR, int GAP, int SRC, int... RS>
 static hipError_t go_fast_t(const LaunchSpec &s, const KArgs &a, hipStream_t st, int *occ_out) {
     const void *fn = reinterpret_cast<const void *>(&pa_fast_kernel<LOC, DIR, GAP, SRC, RS...>);
+    const int block = s.block > 0 && s.block <= FAST_BLOCK && s.block % WAVE == 0 ? s.block : 256;
     if (occ_out) {
         int blocks = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, fn, FAST_BLOCK, s.lds_bytes) != hipSuccess)
-            blocks = 1;
-        *occ_out = blocks * (FAST_BLOCK / WAVE);
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, fn, block, s.lds_bytes) != hipSuccess) blocks = 1;
+        *occ_out = blocks * (block / WAVE);
         return hipSuccess;
     }
-    const int block = s.block > 0 && s.block <= FAST_BLOCK && s.block % WAVE == 0 ? s.block : 256;
     hipLaunchKernelGGL((pa_fast_kernel<LOC, DIR, GAP, SRC, RS...>), dim3(s.grid), dim3(block), s.lds_bytes, st, a);
     return hipGetLastError();
 }
