@@ -1020,7 +1020,10 @@ __device__ __forceinline__ void solve_group_fast(const KArgs &a, const Group &g,
                 tl = int(tp[act ? jc : 0]);
                 above(jc, nxl);
             } else {
-                if (act && j + AHEAD >= 0 && j + AHEAD < lt) tl = int(ct[off_t + j + AHEAD]);
+                // (local alignments over a table too: 50 pairs of up to 95 x 2,067 0.61 ->
+                // 0.56 ms; 16,384 semiglobal binary pairs 0.34 -> 0.37 ms)
+                if (LOCAL && !BINARY) tl = int(tp[act ? inside(j + AHEAD) : 0]);
+                else if (act && j + AHEAD >= 0 && j + AHEAD < lt) tl = int(ct[off_t + j + AHEAD]);
                 if (rd_top && act && j + AHEAD < lt) above(j + AHEAD, nxl);
             }
             if (pend) {  // after the loads: the next wait on them need not wait for it
