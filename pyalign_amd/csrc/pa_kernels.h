@@ -862,7 +862,7 @@ __device__ __forceinline__ bool solve_group(const KArgs &a, const Group &g, cons
 //
 // Bound by VALU issue.  Kernel times on one MI355X: 65,536 local Gotoh pairs of
 // 50 to 2,000 over a table 3.5 ms; 16,384 global affine pairs of 50 to 1,000
-// 0.53 ms (the general kernel's strict folds with long mode 8.6 ms); 16,384
+// 0.48 ms (the general kernel's strict folds with long mode 8.6 ms); 16,384
 // semiglobal affine pairs of 125 x 300 binary symbols 0.29 ms (0.51 ms).
 // ---------------------------------------------------------------------------
 enum { SRC_TABLE = 0, SRC_PAIR = 1, SRC_BINARY = 2 };
@@ -969,7 +969,7 @@ __device__ __forceinline__ void solve_group_fast(const KArgs &a, const Group &g,
         // lane with none reads column 0): a load that may not have left is counted
         // as if it had not, and the wait for the one before it becomes a wait for
         // this step's (220 pairs of up to 8 x 3,550, six groups: 0.69 -> 0.48 ms;
-        // 16,384 pairs of 50 to 1,000: 0.53 -> 0.46 ms).
+        // 16,384 pairs of 50 to 1,000: 0.53 -> 0.48 ms).
         const bool up_on = rd_top && act;
         const float *up = a.border_t, *upP = a.safe + (DIR == DIR_MIN ? 1 : 0);
         if (GLOBAL && up_on) {

@@ -10,8 +10,8 @@
 // host's order (a problem's bands top down, problems interleaved where there
 // are more bands than workgroups), so a band only waits for the band above it,
 // taken earlier by a running workgroup: no circular wait whatever the grid.
-// (2,048 local pairs of 50 to 2,000 with paths, about 600 of them long:
-// 1.4 ms; problem by problem, each ticket counting through the problems' bands,
+// (2,048 local pairs of 50 to 2,000 with paths, 400 to 600 of them long:
+// 1.4 to 1.6 ms; problem by problem, each ticket counting through the problems' bands,
 // 3.6 ms.)
 //
 // Hand-offs.  Inside a strip, lane l's bottom row (D, P) and the column
